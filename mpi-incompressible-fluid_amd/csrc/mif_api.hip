@@ -86,11 +86,8 @@ struct mif_ctx {
   double kappa = 0;
   // spectral solve
   FftPlan plan[3]{};
-  double* W64[3]{};
-  float* W32[3]{};
-  double* H64[3]{};  // half-angle tables of cell-centred axes
-  float* H32[3]{};
-  double* lam[3]{};
+  unsigned char* tables = nullptr;  // every axis table of the solve, one allocation
+  const double* lam[3]{};
   double inv_norm = 1;
   long bp0 = 0, bplane = 0, belems = 0;
   void* B = nullptr;       // packed working buffer (field precision)
@@ -371,16 +368,16 @@ int pressure_solve(mif_ctx* c, mif_field* p, mif_field* const vel[3], double dt,
                    int nhn) {
   T* B = (T*)c->B;
   const SpectralScale sc = scale_of<T>(c);
-  if (!nhn && fft_fast_len(c->plan[0].L)) {
+  if (!nhn && fused_x_pass(c->plan[0])) {
     FusedIO io{vel[0]->data, vel[1]->data, vel[2]->data, p->data, c->L, dt};
     {
       KTimer t(c, MIF_KC_FFT_X_DIV);
-      launch_fft_pow2<T>(c->g, 0, 0, c->plan[0], sc, B, c->bp0, c->bplane, &io, c->stream);
+      launch_fused_x<T>(c->g, 0, c->plan[0], sc, B, c->bp0, c->bplane, io, c->stream);
     }
     spectral_middle<T>(c, B);
     {
       KTimer t(c, MIF_KC_FFT_X_UNPACK);
-      launch_fft_pow2<T>(c->g, 0, 1, c->plan[0], sc, B, c->bp0, c->bplane, &io, c->stream);
+      launch_fused_x<T>(c->g, 1, c->plan[0], sc, B, c->bp0, c->bplane, io, c->stream);
     }
     LAUNCHCHK(c);
     return MIF_OK;
@@ -490,18 +487,18 @@ int pressure_solve_mixed(mif_ctx* c, mif_field* p, mif_field* const vel[3], doub
 // FP32 fields.
 int pressure_solve_mixed64(mif_ctx* c, mif_field* p, mif_field* const vel[3], double dt, const FnDesc& gp, double tg,
                            int nhn) {
-  if (!nhn && fft_fast_len(c->plan[0].L)) {
+  if (!nhn && fused_x_pass(c->plan[0])) {
     FusedIO io{vel[0]->data, vel[1]->data, vel[2]->data, p->data, c->L, dt};
     io.fields_fp32 = 1;
     const SpectralScale sc = scale_of<double>(c);
     {
       KTimer t(c, MIF_KC_FFT_X_DIV);
-      launch_fft_pow2<double>(c->g, 0, 0, c->plan[0], sc, c->B64, c->bp0, c->bplane, &io, c->stream);
+      launch_fused_x<double>(c->g, 0, c->plan[0], sc, c->B64, c->bp0, c->bplane, io, c->stream);
     }
     spectral_middle<double>(c, c->B64);
     {
       KTimer t(c, MIF_KC_FFT_X_UNPACK);
-      launch_fft_pow2<double>(c->g, 0, 1, c->plan[0], sc, c->B64, c->bp0, c->bplane, &io, c->stream);
+      launch_fused_x<double>(c->g, 1, c->plan[0], sc, c->B64, c->bp0, c->bplane, io, c->stream);
     }
     LAUNCHCHK(c);
     return MIF_OK;
@@ -544,7 +541,7 @@ int pressure_solve_mixed_dc1(mif_ctx* c, mif_field* p, mif_field* const vel[3], 
   io.partial = c->xpart;
   {
     KTimer t(c, MIF_KC_FFT_X_DIV);
-    launch_fft_pow2<float>(c->g, 0, 0, c->plan[0], sc, B32, c->bp0, c->bplane, &io, c->stream);
+    launch_fused_x<float>(c->g, 0, c->plan[0], sc, B32, c->bp0, c->bplane, io, c->stream);
   }
   {
     KTimer t(c, MIF_KC_DEFECT);
@@ -563,13 +560,13 @@ int pressure_solve_mixed_dc1(mif_ctx* c, mif_field* p, mif_field* const vel[3], 
     rio.phi32 = B32;
     rio.b64 = c->B64;
     rio.bmean = c->red_b;
-    launch_fft_pow2<float>(c->g, 0, 0, c->plan[0], sc, R32, c->bp0, c->bplane, &rio, c->stream);
+    launch_fused_x<float>(c->g, 0, c->plan[0], sc, R32, c->bp0, c->bplane, rio, c->stream);
   }
   spectral_middle<float>(c, R32);
   io.add32 = B32;
   {
     KTimer t(c, MIF_KC_FFT_X_UNPACK);
-    launch_fft_pow2<float>(c->g, 0, 1, c->plan[0], sc, R32, c->bp0, c->bplane, &io, c->stream);
+    launch_fused_x<float>(c->g, 1, c->plan[0], sc, R32, c->bp0, c->bplane, io, c->stream);
   }
   {
     KTimer t(c, MIF_KC_DEFECT);
@@ -582,7 +579,7 @@ int pressure_solve_mixed_dc1(mif_ctx* c, mif_field* p, mif_field* const vel[3], 
 
 bool dc1_fused(const mif_ctx* c, int nhn) {
   return !is_fp64(c) && !mixed_solve_fp64(c) && c->sweeps == 1 && !nhn && c->nxpart > 0 &&
-         fft_fast_len(c->plan[0].L);
+         fused_x_pass(c->plan[0]);
 }
 
 int pressure_solve_any(mif_ctx* c, mif_field* p, mif_field* const vel[3], double dt, const FnDesc& gp, double tg,
@@ -1021,6 +1018,13 @@ int upload_face_tables(mif_ctx* c, bool velocity, const double* host, int count,
   return MIF_OK;
 }
 
+// Whether an axis has no specialised transform kernel.
+bool dense_axis(int axis, const FftPlan& P) {
+  if (P.dct2 || P.L < 2 || fft_fast_len(P.L)) return false;
+  // the half-length DCT-I of long wall-normal y axes
+  return !(axis == 1 && !P.periodic && (P.L == 1024 || P.L == 1536 || P.L == 2048));
+}
+
 // Constants, layout, transform plans and scratch of a new context.
 int ctx_init(mif_ctx* c, const mif_grid* grid, const uint64_t Ng[3], int precision, int device,
              const int cell[3]) {
@@ -1110,6 +1114,17 @@ int ctx_init(mif_ctx* c, const mif_grid* grid, const uint64_t Ng[3], int precisi
     HIPCHK(nullptr, hipMalloc(&c->red_b, 2 * sizeof(Red3)));
     c->red_phi = c->red_b + 1;
   }
+  // the axis tables, gathered on the host and copied once; `at` remembers
+  // which pointer each one sets
+  std::vector<unsigned char> tab;
+  std::vector<std::pair<const void**, size_t>> at;
+  auto add_table = [&](auto** ptr, const auto& v) {
+    if (v.empty()) return;
+    const size_t off = (tab.size() + 255) / 256 * 256, bytes = v.size() * sizeof(v[0]);
+    tab.resize(off + bytes);
+    std::memcpy(tab.data() + off, v.data(), bytes);
+    at.push_back({(const void**)ptr, off});
+  };
   double norm = 1.0;
   double lam_max = 0, lam_min = 0;  // |lambda| extremes of the 3-D operator
   for (int a = 0; a < 3; a++) {
@@ -1120,45 +1135,47 @@ int ctx_init(mif_ctx* c, const mif_grid* grid, const uint64_t Ng[3], int precisi
     P.dct2 = g.cell[a];
     P.L = g.periodic[a] || g.cell[a] ? n : 2 * (n - 1);
     factor_radices(P.L, P);
+    const bool f32 = precision == MIF_PRECISION_MIXED;
     if (P.dct2) {
       // (cos, sin)(pi k / (2n)) of the DCT-II/III pre- and post-processing
       std::vector<double> h64(2 * (size_t)n);
-      std::vector<float> h32(2 * (size_t)n);
+      std::vector<float> h32(f32 ? 2 * (size_t)n : 0);
       for (int k = 0; k < n; k++) {
         const long double ang = 3.141592653589793238462643383279502884L * (long double)k / (2.0L * n);
-        h64[2 * k] = (double)cosl(ang);
-        h64[2 * k + 1] = (double)sinl(ang);
-        h32[2 * k] = (float)cosl(ang);
-        h32[2 * k + 1] = (float)sinl(ang);
+        const long double cs[2] = {cosl(ang), sinl(ang)};
+        for (int q = 0; q < 2; q++) {
+          h64[2 * k + q] = (double)cs[q];
+          if (f32) h32[2 * k + q] = (float)cs[q];
+        }
       }
-      HIPCHK(nullptr, hipMalloc(&c->H64[a], h64.size() * sizeof(double)));
-      HIPCHK(nullptr, hipMalloc(&c->H32[a], h32.size() * sizeof(float)));
-      HIPCHK(nullptr, hipMemcpy(c->H64[a], h64.data(), h64.size() * sizeof(double), hipMemcpyHostToDevice));
-      HIPCHK(nullptr, hipMemcpy(c->H32[a], h32.data(), h32.size() * sizeof(float), hipMemcpyHostToDevice));
-      P.H64 = c->H64[a];
-      P.H32 = c->H32[a];
+      add_table(&P.H64, h64);
+      add_table(&P.H32, h32);
     }
-    std::vector<double> w64(2 * (size_t)P.L);
-    std::vector<float> w32(2 * (size_t)P.L);
-    for (int e = 0; e < P.L; e++) {
-      const long double ang = 2.0L * 3.141592653589793238462643383279502884L * (long double)e / (long double)P.L;
-      w64[2 * e] = (double)cosl(ang);
-      w64[2 * e + 1] = (double)-sinl(ang);
-      w32[2 * e] = (float)cosl(ang);
-      w32[2 * e + 1] = (float)-sinl(ang);
+    if (dense_axis(a, P) && dense_plan(n, P.periodic, &P.dense)) {
+      std::vector<double> m64(dense_table_elems(P.dense));
+      std::vector<float> m32(f32 ? m64.size() : 0);
+      dense_table(P.dense, m64.data(), f32 ? m32.data() : nullptr);
+      add_table(&P.dense.M64, m64);
+      add_table(&P.dense.M32, m32);
+    } else {
+      std::vector<double> w64(2 * (size_t)P.L);
+      std::vector<float> w32(f32 ? 2 * (size_t)P.L : 0);
+      for (int e = 0; e < P.L; e++) {
+        const long double ang = 2.0L * 3.141592653589793238462643383279502884L * (long double)e / (long double)P.L;
+        const long double cs[2] = {cosl(ang), -sinl(ang)};
+        for (int q = 0; q < 2; q++) {
+          w64[2 * e + q] = (double)cs[q];
+          if (f32) w32[2 * e + q] = (float)cs[q];
+        }
+      }
+      add_table(&P.W64, w64);
+      add_table(&P.W32, w32);
     }
-    HIPCHK(nullptr, hipMalloc(&c->W64[a], w64.size() * sizeof(double)));
-    HIPCHK(nullptr, hipMalloc(&c->W32[a], w32.size() * sizeof(float)));
-    HIPCHK(nullptr, hipMemcpy(c->W64[a], w64.data(), w64.size() * sizeof(double), hipMemcpyHostToDevice));
-    HIPCHK(nullptr, hipMemcpy(c->W32[a], w32.data(), w32.size() * sizeof(float), hipMemcpyHostToDevice));
-    P.W64 = c->W64[a];
-    P.W32 = c->W32[a];
     std::vector<double> lam(n);
     for (int k = 0; k < n; k++)
       lam[k] = g.periodic[a] ? eig_periodic(k, g.h[a], n)
                              : (g.cell[a] ? eig_cell_neumann(k, g.h[a], n) : eig_neumann(k, g.h[a], n));
-    HIPCHK(nullptr, hipMalloc(&c->lam[a], n * sizeof(double)));
-    HIPCHK(nullptr, hipMemcpy(c->lam[a], lam.data(), n * sizeof(double), hipMemcpyHostToDevice));
+    add_table(&c->lam[a], lam);
     double amax = 0, amin = 0;
     for (int k = 0; k < n; k++) {
       const double v = std::fabs(lam[k]);
@@ -1171,6 +1188,9 @@ int ctx_init(mif_ctx* c, const mif_grid* grid, const uint64_t Ng[3], int precisi
     // the DCT-III of a cell-centred axis returns n times the line
     norm *= (double)(Ng[a] - 1) * (g.periodic[a] || g.cell[a] ? 1.0 : 2.0);
   }
+  HIPCHK(nullptr, hipMalloc(&c->tables, tab.size()));
+  HIPCHK(nullptr, hipMemcpy(c->tables, tab.data(), tab.size(), hipMemcpyHostToDevice));
+  for (const auto& e : at) *e.first = c->tables + e.second;
   c->inv_norm = 1.0 / norm;
   c->kappa = lam_min > 0 ? lam_max / lam_min : 0;
   if (precision == MIF_PRECISION_MIXED) {
@@ -1306,13 +1326,7 @@ int mif_ctx_destroy(mif_ctx* c) {
   (void)hipFree(c->adj_partial);
   (void)hipFree(c->adj_fbar);
   (void)hipFree(c->trig);
-  for (int a = 0; a < 3; a++) {
-    (void)hipFree(c->W64[a]);
-    (void)hipFree(c->W32[a]);
-    (void)hipFree(c->H64[a]);
-    (void)hipFree(c->H32[a]);
-    (void)hipFree(c->lam[a]);
-  }
+  (void)hipFree(c->tables);
   (void)hipFree(c->staging);
   (void)hipFree(c->partial);
   (void)hipFree(c->red_out);

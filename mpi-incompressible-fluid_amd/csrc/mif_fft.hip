@@ -1,4 +1,6 @@
-// mif_fft.hip -- LDS transform kernels of the spectral Poisson solve.
+// mif_fft.hip -- LDS transform kernels of the spectral Poisson solve, for the
+// line lengths that neither mif_fft_pow2.hip nor mif_dense.hip covers, and the
+// choice between the three.
 //
 // The reference solves L phi = b by diagonalisation: a real transform along
 // every axis (FFTW_REDFT00 = DCT-I on Neumann axes, FFTW_R2HC / FFTW_HC2R on
@@ -391,6 +393,10 @@ void launch_fft_axis(const DGrid& g, int axis, int dir, int fused, const FftPlan
     return;
   }
   if (plan.L >= 2 && launch_fft_pow2<T>(g, axis, mode, plan, sc, B, bp0, bplane, nullptr, st)) return;
+  if (plan.dense.M64) {
+    launch_dense<T>(g, axis, mode, plan.dense, sc, B, bp0, bplane, nullptr, st);
+    return;
+  }
   if (axis == 0) {
     if (mode == 0) launch_one<T, 0, 0>(g, plan, sc, B, bp0, bplane, st);
     else launch_one<T, 0, 1>(g, plan, sc, B, bp0, bplane, st);
@@ -398,12 +404,23 @@ void launch_fft_axis(const DGrid& g, int axis, int dir, int fused, const FftPlan
     if (mode == 0) launch_one<T, 1, 0>(g, plan, sc, B, bp0, bplane, st);
     else launch_one<T, 1, 1>(g, plan, sc, B, bp0, bplane, st);
   } else {
-    if (mode == 0) launch_one<T, 2, 0>(g, plan, sc, B, bp0, bplane, st);
-    else if (mode == 1) launch_one<T, 2, 1>(g, plan, sc, B, bp0, bplane, st);
-    else launch_one<T, 2, 2>(g, plan, sc, B, bp0, bplane, st);
+    launch_one<T, 2, 2>(g, plan, sc, B, bp0, bplane, st);
   }
 }
 
+bool fused_x_pass(const FftPlan& plan) { return fft_fast_len(plan.L) || plan.dense.M64; }
+
+template <typename T>
+void launch_fused_x(const DGrid& g, int mode, const FftPlan& plan, const SpectralScale& sc, T* B, long bp0, long bplane,
+                    const FusedIO& io, hipStream_t st) {
+  if (launch_fft_pow2<T>(g, 0, mode, plan, sc, B, bp0, bplane, &io, st)) return;
+  launch_dense<T>(g, 0, mode, plan.dense, sc, B, bp0, bplane, &io, st);
+}
+
+template void launch_fused_x<double>(const DGrid&, int, const FftPlan&, const SpectralScale&, double*, long, long,
+                                     const FusedIO&, hipStream_t);
+template void launch_fused_x<float>(const DGrid&, int, const FftPlan&, const SpectralScale&, float*, long, long,
+                                    const FusedIO&, hipStream_t);
 template void launch_fft_axis<double>(const DGrid&, int, int, int, const FftPlan&, const SpectralScale&, double*, long,
                                       long, hipStream_t);
 template void launch_fft_axis<float>(const DGrid&, int, int, int, const FftPlan&, const SpectralScale&, float*, long,

@@ -1182,7 +1182,7 @@ int fused_x_blocks(const DGrid& g, const FftPlan& plan, bool fp64) {
     case 384: np = np_x(fp64, 384); break;
     case 768: np = np_x(fp64, 768); break;
     case 1024: case 1536: np = 1; break;
-    default: return 0;
+    default: return plan.dense.M64 ? dense_x_blocks(g) : 0;
   }
   const long lines = (long)g.npts[1] * g.npts[2];
   return (int)((lines + 2 * np - 1) / (2 * np));

@@ -48,6 +48,17 @@ struct Red3 {
   double s1, s2, mx;
 };
 
+// One axis as products with the transform's matrices (mif_dense.hip), for
+// lengths without a specialised kernel: R is the mirror length (n, or n - 1 on
+// a Neumann axis), H = R/2 + 1 the rows of the folded line, MT and KS its
+// 16-row and 8-column tiles, M the fragment tables (null: no dense pass).
+struct DensePlan {
+  int n, R, H, MT, KS;
+  int periodic;
+  const double* M64;
+  const float* M32;
+};
+
 // One axis of the spectral Poisson solve: complex transform length L (= n on
 // a periodic axis, 2(n-1) on a Neumann axis), its radix factorisation and
 // the twiddle table W[e] = exp(-2 pi i e / L).
@@ -63,6 +74,7 @@ struct FftPlan {
   int dct2;
   const double* H64;
   const float* H32;
+  DensePlan dense;
 };
 
 // Scaling applied between the forward and inverse transform of the last
@@ -203,6 +215,24 @@ bool fft_fast_len(int L);
 template <typename T>
 bool launch_fft_pow2(const DGrid& g, int axis, int mode, const FftPlan& plan, const SpectralScale& sc, T* B, long bp0,
                      long bplane, const FusedIO* io, hipStream_t st);
+// The passes as matrix products (mif_dense.hip): axis 0 with mode 0 / 1 (io
+// as in launch_fft_pow2), axis 1 with mode 0 / 1, axis 2 with mode 2.
+// dense_plan fills the tile counts (false: the line is too long).
+bool dense_plan(int n, bool periodic, DensePlan* P);
+// The fragment tables of a plan: dense_table_elems elements, in FP64 and (out32
+// not null) FP32.
+size_t dense_table_elems(const DensePlan& P);
+void dense_table(const DensePlan& P, double* out64, float* out32);
+template <typename T>
+void launch_dense(const DGrid& g, int axis, int mode, const DensePlan& P, const SpectralScale& sc, T* B, long bp0,
+                  long bplane, const FusedIO* io, hipStream_t st);
+int dense_x_blocks(const DGrid& g);
+// Whether the axis-0 pass of a plan has a form fused with the divergence and
+// the unpack, and that pass (mode 0 forward, 1 inverse).
+bool fused_x_pass(const FftPlan& plan);
+template <typename T>
+void launch_fused_x(const DGrid& g, int mode, const FftPlan& plan, const SpectralScale& sc, T* B, long bp0, long bplane,
+                    const FusedIO& io, hipStream_t st);
 // Workgroups of the specialised x pass of a plan (0 without a kernel): the
 // number of partial sums a fused x pass with FusedIO::dc leaves.
 int fused_x_blocks(const DGrid& g, const FftPlan& plan, bool fp64);
