@@ -124,7 +124,8 @@ struct StageTile {
   static constexpr int PQ = (PLANE_ELEMS + STN - 1) / STN;   // plane elements per thread
   static_assert(STN == 512, "the stage kernel's launch bounds");
 };
-// planes per workgroup.  FP32 on 128 x 4 tiles at 256^3: 8 planes 180.4 us,
+// planes per workgroup on large grids (stage_chunk takes fewer on small
+// ones).  FP32 on 128 x 4 tiles at 256^3: 8 planes 180.4 us,
 // 16 176.5 us, 24 178.0 us, 32 192.5 us.  FP64 on 64 x 8 tiles, with the
 // plane order of k_stage: 4 planes 329 us, 6 328, 8 320, 10 320,
 // 12 323, 16 336, 24 357, 32 342 (four ring slots instead of three: 8 planes
@@ -168,7 +169,7 @@ template <typename T, int KIND, bool FT = false, bool NT = false, bool VEC = fal
 __global__ void __launch_bounds__(512)
 __attribute__((amdgpu_waves_per_eu(KIND <= 3 && (sizeof(T) == 8 || PROJ) ? (sizeof(T) == 8 && PROJ ? 4 : 6)
                                                                       : (FT && sizeof(T) == 4 ? 6 : 1))))
-k_stage(DGrid g, Layout L, StageArgs s, VelStageArgs vs, int imax, int jmax, int kmax, int ntx, int nty, int ntiles) {
+k_stage(DGrid g, Layout L, StageArgs s, VelStageArgs vs, int imax, int jmax, int kmax, int ntx, int nty, int ntiles, int kchunk) {
   static_assert(!PROJ || KIND <= 3, "a fused projection belongs to the full-step kinds");
   // ring slots: 3 (planes k-1, k, k+1; two barriers per plane) or 4 and
   // more (plane k+2 is committed into a free slot while plane k is
@@ -191,9 +192,8 @@ k_stage(DGrid g, Layout L, StageArgs s, VelStageArgs vs, int imax, int jmax, int
   const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * STX + tx;
   const int tile = xcd_tile(blockIdx.x, ntiles);
   const int bx = tile % ntx, by = (tile / ntx) % nty, bz = tile / (ntx * nty);
-  constexpr int SKB = stage_planes<T, KIND, NT, PROJ>();
-  const int i0 = bx * STX + 1, j0 = by * STY + 1, k0 = bz * SKB + 1;
-  const int k1 = min(k0 + SKB, kmax + 1);
+  const int i0 = bx * STX + 1, j0 = by * STY + 1, k0 = bz * kchunk + 1;
+  const int k1 = min(k0 + kchunk, kmax + 1);
   const int i = i0 + tx, j = j0 + ty;
   const T* X[3];
   for (int f = 0; f < 3; f++) X[f] = (const T*)(KIND <= 3 ? s.X[f] : vs.X[f]);
@@ -1165,6 +1165,23 @@ __global__ void __launch_bounds__(256) k_reduce_final(const Red3* partial, int n
 // ---------------------------------------------------------------------------
 // Host launchers.
 // ---------------------------------------------------------------------------
+// Planes per workgroup of a stage kernel: `most` (stage_planes) on grids that
+// fill the device at that, fewer on smaller ones, where a workgroup's planes
+// are a serial chain (about 2.4 us each in FP64) while compute units idle.
+// cols: tiles of a plane.  Up to three planes while the tiles then fit one
+// per CU, beyond that the chunk that gives 2 3/4 workgroups per CU: just over
+// two per CU (the resident set) the second round runs nearly empty.  Stage
+// launch, most -> this rule, FP64 / FP32 (us): 32 x 32 x 64 nodes 30.5 -> 9.8 /
+// 24.7 -> 9.6 (one / two planes); 64^3 32.1 -> 14.7 / 27.0 -> 13.7 (three); 96^3
+// 32.3 -> 26.4 / 27.3 -> 17.7 (three; four: 30.0 / 19.4, eight: 32.1 / 21.7);
+// 128^3 55.4 -> 46.6 / 37.9 -> 27.2 (six; eight: 53.4 / 31.8); 180 x 102 x 150
+// 68.3 -> 68.2 (eight); from 192^3 on the rule gives `most`.
+static int stage_chunk(long cols, int planes, int most) {
+  const long all = cols * planes;
+  const long c = all <= 3 * 256 ? (all + 255) / 256 : max(3L, (all + 352) / 704);
+  return (int)min((long)most, c);
+}
+
 template <typename T, int KIND, bool FT = false, bool NT = false>
 static void launch_stage_kind(const DGrid& g, const Layout& L, const StageArgs& s, const VelStageArgs& vs,
                               hipStream_t st) {
@@ -1181,9 +1198,9 @@ static void launch_stage_kind(const DGrid& g, const Layout& L, const StageArgs& 
   const dim3 blk(STX, STY, 1);
   auto go = [&](auto vec, auto proj) {
     constexpr bool V = decltype(vec)::value, P = decltype(proj)::value;
-    constexpr int SKB = stage_planes<T, KIND, NT, P>();
-    const int ntiles = ntx * nty * ((kmax + SKB - 1) / SKB);
-    k_stage<T, KIND, FT, NT, V, P><<<ntiles, blk, 0, st>>>(g, L, s, vs, imax, jmax, kmax, ntx, nty, ntiles);
+    const int kchunk = stage_chunk(ntx * nty, kmax, stage_planes<T, KIND, NT, P>());
+    const int ntiles = ntx * nty * ((kmax + kchunk - 1) / kchunk);
+    k_stage<T, KIND, FT, NT, V, P><<<ntiles, blk, 0, st>>>(g, L, s, vs, imax, jmax, kmax, ntx, nty, ntiles, kchunk);
   };
   using yes = std::true_type;
   using no = std::false_type;
