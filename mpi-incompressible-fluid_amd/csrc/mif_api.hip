@@ -116,10 +116,10 @@ struct mif_ctx {
   double* adj_partial = nullptr;
   double* adj_fbar = nullptr;
   bool adj_ready = false;  // every adjoint buffer allocated
-  // velocity-only step: sin/cos of the coordinates of every axis,
-  // unshifted and staggered (launch_trig_tables), filled on first use
-  double* trig = nullptr;
-  int trig_n = 0;
+  // functions of one coordinate that the boundary data, the forcing and the
+  // Neumann data are built from (launch_axis_tables)
+  double* axis = nullptr;
+  int axis_n = 0;
   // transfers and reductions
   double* staging = nullptr;
   long staging_elems = 0;
@@ -267,6 +267,14 @@ double eig_cell_neumann(size_t index, double delta, size_t N) {
 template <typename T>
 T* fptr(mif_field* f) {
   return (T*)f->data;
+}
+
+// A descriptor with the context's axis tables.
+FnDesc fn_of(const mif_ctx* c, const mif_function* f) {
+  FnDesc d = make_fn(f);
+  d.axis = c->axis;
+  d.an = c->axis_n;
+  return d;
 }
 
 bool is_fp64(const mif_ctx* c) { return c->precision == MIF_PRECISION_FP64; }
@@ -803,16 +811,6 @@ int velocity_timestep(mif_ctx* c, mif_field* const vel[3], mif_field* const buf[
   VelStageArgs s{};
   s.dt = dt;
   s.forcing = fo;
-  if (fo.kind == MIF_FN_VT_FORCING) {
-    if (!c->trig) {
-      const int tn = std::max(c->g.N[0], std::max(c->g.N[1], c->g.N[2])) + 1;
-      HIPCHK(c, hipMalloc(&c->trig, 12 * (size_t)tn * sizeof(double)));
-      c->trig_n = tn;
-      launch_trig_tables(c->g, c->trig, tn, c->stream);
-    }
-    s.trig = c->trig;
-    s.tn = c->trig_n;
-  }
   for (int q = 0; q < 3; q++) {
     s.V[q] = vel[q]->data;
     s.R[q] = rhs[q]->data;
@@ -1197,6 +1195,11 @@ int ctx_init(mif_ctx* c, const mif_grid* grid, const uint64_t Ng[3], int precisi
     c->nxpart = fused_x_blocks(g, c->plan[0], false);
     if (c->nxpart > 0) HIPCHK(nullptr, hipMalloc(&c->xpart, c->nxpart * sizeof(Red3)));
   }
+  // the largest index the closed forms take is one past the largest extent
+  c->axis_n = std::max(g.N[0], std::max(g.N[1], g.N[2])) + 2;
+  HIPCHK(nullptr, hipMalloc(&c->axis, axis_index(3, 0, 0, c->axis_n) * sizeof(double)));
+  launch_axis_tables(g, c->axis, c->axis_n, c->stream);
+  LAUNCHCHK(nullptr);
   // transfers and reductions
   long mx = 0;
   for (int s = 0; s < 4; s++) {
@@ -1325,7 +1328,7 @@ int mif_ctx_destroy(mif_ctx* c) {
   (void)hipFree(c->ftab);
   (void)hipFree(c->adj_partial);
   (void)hipFree(c->adj_fbar);
-  (void)hipFree(c->trig);
+  (void)hipFree(c->axis);
   (void)hipFree(c->tables);
   (void)hipFree(c->staging);
   (void)hipFree(c->partial);
@@ -1516,7 +1519,7 @@ int mif_field_set(mif_field* f, const mif_function* fn, int comp, double t, int 
   if (!f || !f->ctx || !fn) return fail(f ? f->ctx : nullptr, MIF_ERR_INVALID_ARGUMENT, "null argument");
   mif_ctx* c = f->ctx;
   if (comp < 0 || comp > 2) return fail(c, MIF_ERR_INVALID_ARGUMENT, "component %d", comp);
-  const FnDesc d = make_fn(fn);
+  const FnDesc d = fn_of(c, fn);
   if (is_fp64(c))
     launch_set<double>(c->g, c->L, fptr<double>(f), f->stag, comp, d, t, include_border, c->stream);
   else
@@ -1541,7 +1544,7 @@ int mif_velocity_apply_bc(mif_field* const vel[3], const mif_function* fn, doubl
   int rc = check_vel(vel, &c);
   if (rc) return rc;
   if (!fn) return fail(c, MIF_ERR_INVALID_ARGUMENT, "null function");
-  const FnDesc d = make_fn(fn);
+  const FnDesc d = fn_of(c, fn);
   if (is_fp64(c))
     apply_bc<double>(c, vel, d, t);
   else
@@ -1601,7 +1604,7 @@ int mif_timestep(mif_field* const vel[3], mif_field* const buf[3], mif_field* co
   int rc = check_timestep(vel, buf, buf2, p, pb, false, &c);
   if (rc) return rc;
   if (!exact_velocity) return fail(c, MIF_ERR_INVALID_ARGUMENT, "null exact velocity");
-  const FnDesc d = make_fn(exact_velocity);
+  const FnDesc d = fn_of(c, exact_velocity);
   const FnDesc ev[3] = {d, d, d};
   return run_timestep(c, vel, buf, buf2, ev, nullptr, t_n, p, pb);
 }
@@ -1613,7 +1616,7 @@ int mif_timestep_n(mif_field* const vel[3], mif_field* const buf[3], mif_field* 
   if (rc) return rc;
   if (!exact_velocity) return fail(c, MIF_ERR_INVALID_ARGUMENT, "null exact velocity");
   if (nsteps < 0) return fail(c, MIF_ERR_INVALID_ARGUMENT, "negative step count %d", nsteps);
-  const FnDesc d = make_fn(exact_velocity);
+  const FnDesc d = fn_of(c, exact_velocity);
   const FnDesc ev[3] = {d, d, d};
   StepCarry cs;
   for (int s = 0; s < nsteps; s++) {
@@ -1633,14 +1636,14 @@ int mif_timestep_nhn(mif_field* const vel[3], mif_field* const buf[3], mif_field
   int rc = check_timestep(vel, buf, buf2, p, pb, true, &c);
   if (rc) return rc;
   if (!exact_velocity || !exact_grad_p) return fail(c, MIF_ERR_INVALID_ARGUMENT, "null function");
-  const FnDesc d = make_fn(exact_velocity);
+  const FnDesc d = fn_of(c, exact_velocity);
   const FnDesc ev[3] = {d, d, d};
   // TimeVectorFunction::get_difference_over_time(new_time, prev_time) yields
   // f(prev_time) - f(new_time) (src/Timestep.cpp:89-95, src/VectorFunction.cpp:53-61)
   const StageTimes st = stage_times(c->g.dt, t_n);
   FnDesc gd[3];
   for (int s = 0; s < 3; s++) {
-    gd[s] = make_fn(exact_grad_p);
+    gd[s] = fn_of(c, exact_grad_p);
     gd[s].base = exact_grad_p->kind;
     gd[s].kind = MIF_FN_TIME_DIFFERENCE;
     gd[s].t0 = st.time[s + 1];
@@ -1682,9 +1685,9 @@ static int velocity_timestep_any(mif_field* const vel[3], mif_field* const buf[3
   if (faces) {
     if ((rc = upload_face_tables(c, true, faces, 3, d))) return rc;
   } else {
-    d[0] = d[1] = d[2] = make_fn(ev);
+    d[0] = d[1] = d[2] = fn_of(c, ev);
   }
-  const FnDesc f = make_fn(fo);
+  const FnDesc f = fn_of(c, fo);
   if (is_fp64(c)) return velocity_timestep<double>(c, vel, buf, rhs, d, f, t_n);
   return velocity_timestep<float>(c, vel, buf, rhs, d, f, t_n);
 }
@@ -1719,7 +1722,7 @@ int mif_solve_pressure_non_homogeneous_neumann(mif_field* p, mif_field* const ve
     return fail(c, MIF_ERR_INVALID_ARGUMENT, "bad pressure field or gradient");
   if (c->g.periodic[0] || c->g.periodic[1] || c->g.periodic[2])
     return fail(c, MIF_ERR_INVALID_ARGUMENT, "non-homogeneous Neumann data needs walls on every axis");
-  const FnDesc d = make_fn(gp);
+  const FnDesc d = fn_of(c, gp);
   return pressure_solve_any(c, p, vel, dt, d, t, 1);
 }
 
@@ -1875,7 +1878,7 @@ bool is_node_field_of(const mif_field* f, const mif_ctx* c) {
 int mif_adjust_pressure(mif_field* p, const mif_function* fn, double t) {
   if (!p || !p->ctx || !fn || p->stag != MIF_STAGGER_NONE)
     return fail(p ? p->ctx : nullptr, MIF_ERR_INVALID_ARGUMENT, "bad arguments");
-  return adjust_pressure_impl(p->ctx, p, make_fn(fn), t, ExactTables{});
+  return adjust_pressure_impl(p->ctx, p, fn_of(p->ctx, fn), t, ExactTables{});
 }
 
 int mif_adjust_pressure_tabulated(mif_field* p, const mif_field* exact) {
@@ -1891,7 +1894,7 @@ int mif_error_norms_velocity(mif_field* const vel[3], const mif_function* fn, do
   int rc = check_vel(vel, &c);
   if (rc) return rc;
   if (!fn || !out) return fail(c, MIF_ERR_INVALID_ARGUMENT, "null argument");
-  return norms_velocity_impl(c, vel, make_fn(fn), t, ExactTables{}, out);
+  return norms_velocity_impl(c, vel, fn_of(c, fn), t, ExactTables{}, out);
 }
 
 int mif_error_norms_velocity_tabulated(mif_field* const vel[3], mif_field* const exact[3], double out[3]) {
@@ -1911,7 +1914,7 @@ int mif_error_norms_velocity_tabulated(mif_field* const vel[3], mif_field* const
 int mif_error_norms_pressure(const mif_field* p, const mif_function* fn, double t, double out[3]) {
   if (!p || !p->ctx || !fn || !out || p->stag != MIF_STAGGER_NONE)
     return fail(p ? p->ctx : nullptr, MIF_ERR_INVALID_ARGUMENT, "bad arguments");
-  return norms_pressure_impl(p->ctx, p, make_fn(fn), t, ExactTables{}, out);
+  return norms_pressure_impl(p->ctx, p, fn_of(p->ctx, fn), t, ExactTables{}, out);
 }
 
 int mif_error_norms_pressure_tabulated(const mif_field* p, const mif_field* exact, double out[3]) {

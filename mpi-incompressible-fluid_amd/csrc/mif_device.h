@@ -12,6 +12,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <cmath>
+
 #include "../../include/mif_types.h"
 
 namespace mif {
@@ -69,7 +71,18 @@ struct FnDesc {
   double Re, c[3], t0, t1;
   const double* tab;
   long toff[3][6];
+  // the context's axis tables (AxisTab), for the closed forms that separate
+  // into functions of one coordinate
+  const double* axis;
+  int an;
 };
+
+// Functions of one coordinate tabulated per axis at its unstaggered (sh = 0)
+// and staggered (sh = 1, shifted by -h/2) indices i < n, in FP64: entry
+// ((a * 2 + sh) * kAxisFns + fn) * n + i.  EXP_A, SIN_A, COS_A take (pi/4) x
+// and SIN_D, COS_D (pi/2) x, the Ethier-Steinman arguments.
+enum AxisFn { AX_SIN, AX_COS, AX_EXP_A, AX_SIN_A, AX_COS_A, AX_SIN_D, AX_COS_D, kAxisFns };
+__host__ __device__ inline long axis_index(int a, int sh, int fn, int n) { return ((a * 2 + sh) * kAxisFns + fn) * (long)n; }
 
 // Index of point (i, j, k) in the plane of face f (0,1 = z-,z+; 2,3 =
 // y-,y+; 4,5 = x-,x+) of a field with extents e.
@@ -192,6 +205,58 @@ __device__ inline double coord(const DGrid& g, int a, int s, int i) {
   double x = g.min[a] + g.h[a] * (double)(g.base[a] + i);
   if (a == s) x = x - g.h_over_2[a];
   return x;
+}
+
+// Ethier-Steinman field and pressure gradient, and the velocity-only field,
+// from the axis tables, without their factor in time (time_factor).  A sine or
+// cosine of a sum of two coordinates is expanded by the addition theorem, so
+// a value costs table reads and a few products.  s: staggering, c: component.
+struct AxisEval {
+  const double* tab;
+  int n, s, idx[3];
+  __device__ inline double operator()(int a, int fn) const {
+    const int i = a == 0 ? idx[0] : (a == 1 ? idx[1] : idx[2]);
+    return tab[axis_index(a, a == s ? 1 : 0, fn, n) + i];
+  }
+  // sin and cos of (pi/4) x_a + (pi/2) x_b
+  __device__ inline double sin_ad(int a, int b) const {
+    return (*this)(a, AX_SIN_A) * (*this)(b, AX_COS_D) + (*this)(a, AX_COS_A) * (*this)(b, AX_SIN_D);
+  }
+  __device__ inline double cos_ad(int a, int b) const {
+    return (*this)(a, AX_COS_A) * (*this)(b, AX_COS_D) - (*this)(a, AX_SIN_A) * (*this)(b, AX_SIN_D);
+  }
+  // es_u, es_dpdx with (x, y, z) = axes (p, q, r)
+  __device__ inline double es_velocity(int p, int q, int r) const {
+    return -(MIF_PI / 4) * ((*this)(p, AX_EXP_A) * sin_ad(q, r) + (*this)(r, AX_EXP_A) * cos_ad(p, q));
+  }
+  __device__ inline double es_grad_p(int p, int q, int r) const {
+    const double a = MIF_PI / 4, d = MIF_PI / 2;
+    const double ex = (*this)(p, AX_EXP_A), ey = (*this)(q, AX_EXP_A), ez = (*this)(r, AX_EXP_A);
+    const double S1 = sin_ad(p, q), C1 = cos_ad(r, p), S2 = sin_ad(q, r), C2 = cos_ad(p, q), S3 = sin_ad(r, p),
+                 C3 = cos_ad(q, r);
+    const double v = 2 * a * (ex * ex) + 2 * (ey * ez) * (a * C2 * C1 - d * S1 * S3) +
+                     2 * a * (ez * ex) * S2 * (C2 - S1) + 2 * (ex * ey) * C3 * (d * C1 + a * S3);
+    return -a * a / 2 * v;
+  }
+  __device__ inline double vt_velocity(int c) const {
+    if (c == 0) return (*this)(0, AX_SIN) * (*this)(1, AX_COS) * (*this)(2, AX_SIN);
+    if (c == 1) return (*this)(0, AX_COS) * (*this)(1, AX_SIN) * (*this)(2, AX_SIN);
+    return 2 * (*this)(0, AX_COS) * (*this)(1, AX_COS) * (*this)(2, AX_COS);
+  }
+};
+
+// The factor in time of those forms (their only dependence on it).
+__host__ inline double time_factor(int kind, double t, double Re) {
+  const double d = MIF_PI / 2;
+  if (kind == MIF_FN_ES_VELOCITY) return std::exp(-d * d * t / Re);
+  if (kind == MIF_FN_ES_GRAD_P) return std::exp(-2 * d * d * t / Re);
+  return std::sin(t);  // MIF_FN_VT_VELOCITY
+}
+// The factor of the Ethier-Steinman gradient's difference between two times,
+// without the cancellation of two nearly equal exponentials.
+__host__ inline double grad_p_factor_difference(double t1, double t0, double Re) {
+  const double d = MIF_PI / 2;
+  return std::exp(-2 * d * d * t0 / Re) * std::expm1(-2 * d * d * (t1 - t0) / Re);
 }
 
 __device__ inline double eval_at(const DGrid& g, const FnDesc& f, int s, int c, double t, int i, int j, int k) {

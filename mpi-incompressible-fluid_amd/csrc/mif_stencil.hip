@@ -547,11 +547,9 @@ k_stage(DGrid g, Layout L, StageArgs s, VelStageArgs vs, int imax, int jmax, int
           double fc;
           if constexpr (FT) {
             // component c sits at coordinates shifted on axis c
-            const double* tb = vs.trig;
-            const int tn = vs.tn;
-            auto tab = [&](int a, int q, int idx) { return tb[((a * 2 + (a == c ? 1 : 0)) * 2 + q) * tn + idx]; };
-            fc = vt_forcing(c, tab(0, 0, i), tab(0, 1, i), tab(1, 0, j), tab(1, 1, j), tab(2, 0, k), tab(2, 1, k),
-                            sin(vs.t), cos(vs.t), vs.forcing.Re);
+            const AxisEval at{vs.forcing.axis, vs.forcing.an, c, {i, j, k}};
+            fc = vt_forcing(c, at(0, AX_SIN), at(0, AX_COS), at(1, AX_SIN), at(1, AX_COS), at(2, AX_SIN),
+                            at(2, AX_COS), sin(vs.t), cos(vs.t), vs.forcing.Re);
           } else {
             fc = eval_at(g, vs.forcing, c, c, vs.t, i, j, k);
           }
@@ -666,30 +664,33 @@ __global__ void __launch_bounds__(256) k_p_rim(DGrid g, Layout L, const T* __res
                  kmax);
 }
 
-__device__ inline double face_value(const DGrid& g, const FnDesc& f, double t, int c, int face, int i, int j, int k) {
+// Boundary value of component c at point (i, j, k) of a face; ev(s, c, i, j, k)
+// is component c of the exact velocity at the point of staggering s.
+template <typename Ev>
+__device__ inline double face_value(const DGrid& g, Ev ev, int c, int face, int i, int j, int k) {
   // faces 0,1 = z-,z+; 2,3 = y-,y+; 4,5 = x-,x+
   const int axis = 2 - (face >> 1);
-  if (axis != c) return eval_at(g, f, c, c, t, i, j, k);  // tangential: exact value
+  if (axis != c) return ev(c, c, i, j, k);  // tangential: exact value
   const bool hi = face & 1;
   if (c == 2) {
     const int kn = hi ? g.N[2] - 1 : 0;
-    const double wb = eval_at(g, f, 3, 2, t, i, j, kn);
-    const double du_dx = (eval_at(g, f, 0, 0, t, i + 1, j, kn) - eval_at(g, f, 0, 0, t, i, j, kn)) * g.one_over_h[0];
-    const double dv_dy = (eval_at(g, f, 1, 1, t, i, j + 1, kn) - eval_at(g, f, 1, 1, t, i, j, kn)) * g.one_over_h[1];
+    const double wb = ev(3, 2, i, j, kn);
+    const double du_dx = (ev(0, 0, i + 1, j, kn) - ev(0, 0, i, j, kn)) * g.one_over_h[0];
+    const double dv_dy = (ev(1, 1, i, j + 1, kn) - ev(1, 1, i, j, kn)) * g.one_over_h[1];
     return hi ? wb - g.h_over_2[2] * (du_dx + dv_dy) : wb + g.h_over_2[2] * (du_dx + dv_dy);
   }
   if (c == 1) {
     const int jn = hi ? g.N[1] - 1 : 0;
-    const double vb = eval_at(g, f, 3, 1, t, i, jn, k);
-    const double du_dx = (eval_at(g, f, 0, 0, t, i + 1, jn, k) - eval_at(g, f, 0, 0, t, i, jn, k)) * g.one_over_h[0];
-    const double dw_dz = (eval_at(g, f, 2, 2, t, i, jn, k + 1) - eval_at(g, f, 2, 2, t, i, jn, k)) * g.one_over_h[2];
+    const double vb = ev(3, 1, i, jn, k);
+    const double du_dx = (ev(0, 0, i + 1, jn, k) - ev(0, 0, i, jn, k)) * g.one_over_h[0];
+    const double dw_dz = (ev(2, 2, i, jn, k + 1) - ev(2, 2, i, jn, k)) * g.one_over_h[2];
     return hi ? vb - g.h_over_2[1] * (du_dx + dw_dz) : vb + g.h_over_2[1] * (du_dx + dw_dz);
   }
   // c == 0; the x+ wall node is Nx_domains = Nx_global - 1, derivatives at Nx - 1
   const int in = hi ? g.N[0] - 1 : 0;
-  const double ub = eval_at(g, f, 3, 0, t, hi ? g.Ng[0] - 1 : 0, j, k);
-  const double dv_dy = (eval_at(g, f, 1, 1, t, in, j + 1, k) - eval_at(g, f, 1, 1, t, in, j, k)) * g.one_over_h[1];
-  const double dw_dz = (eval_at(g, f, 2, 2, t, in, j, k + 1) - eval_at(g, f, 2, 2, t, in, j, k)) * g.one_over_h[2];
+  const double ub = ev(3, 0, hi ? g.Ng[0] - 1 : 0, j, k);
+  const double dv_dy = (ev(1, 1, in, j + 1, k) - ev(1, 1, in, j, k)) * g.one_over_h[1];
+  const double dw_dz = (ev(2, 2, in, j, k + 1) - ev(2, 2, in, j, k)) * g.one_over_h[2];
   return hi ? ub - g.h_over_2[0] * (dv_dy + dw_dz) : ub + g.h_over_2[0] * (dv_dy + dw_dz);
 }
 
@@ -697,14 +698,37 @@ struct BCArgs {
   void* F[3];
   FnDesc f;
   double t;
+  double tf;        // time_factor (BC_ES, BC_VT)
   int count[3][3];  // threads (opposite shell points) per (component, face pair)
 };
 
 // Face data of a boundary pass: BC_ZERO homogeneous data (no-slip walls),
 // every face value is 0 and the function evaluation code is compiled out,
-// which keeps the kernel small; BC_FN closed-form descriptors evaluated on
-// the device; BC_TABLE values evaluated on the host (FnDesc kFnFaceTable).
-enum BCMode { BC_ZERO = 0, BC_FN = 1, BC_TABLE = 2 };
+// which keeps the kernel small; BC_TABLE values evaluated on the host (FnDesc
+// kFnFaceTable); BC_ES, BC_VT the Ethier-Steinman and velocity-only fields
+// from the axis tables; BC_LID the lid-driven data (one comparison); BC_FN
+// any other closed form through the general evaluator, whose serial chain of
+// FP64 transcendentals (up to ten evaluations per thread) took 30 us on 65^3
+// nodes and 25 us on 96^3 for Ethier-Steinman data (6.7 and 7.1 us from the
+// tables), 63 us on 256^3 for the velocity-only field (16 us) and 12 us on
+// 32 x 32 x 64 for the lid.
+enum BCMode { BC_ZERO = 0, BC_FN = 1, BC_TABLE = 2, BC_ES = 3, BC_VT = 4, BC_LID = 5 };
+
+// Component c of the boundary velocity at point (i, j, k) of staggering s.
+template <int MODE>
+__device__ inline double bc_eval(const DGrid& g, const FnDesc& f, double t, double tf, int s, int c, int i, int j,
+                                 int k) {
+  if constexpr (MODE == BC_ES || MODE == BC_VT) {
+    const AxisEval at{f.axis, f.an, s, {i, j, k}};
+    if constexpr (MODE == BC_VT) return at.vt_velocity(c) * tf;
+    return (c == 0 ? at.es_velocity(0, 1, 2) : (c == 1 ? at.es_velocity(1, 2, 0) : at.es_velocity(2, 0, 1))) * tf;
+  } else if constexpr (MODE == BC_LID) {
+    const double x = coord(g, 0, s, i), xl = f.kind == MIF_FN_LID_1 ? 1.0 : -0.5, eps = 1e-12;
+    return c == 1 && x < xl + eps && x > xl - eps ? 1.0 : 0.0;
+  } else {
+    return eval_at(g, f, s, c, t, i, j, k);
+  }
+}
 
 // Value of shell point (i, j, k) of component c: a Dirichlet face value, or
 // the value at its periodic source, which is then an interior point that
@@ -741,7 +765,9 @@ __device__ inline T shell_value(const DGrid& g, const Layout& L, const BCArgs& a
     else if constexpr (MODE == BC_TABLE)
       return (T)a.f.tab[a.f.toff[c][face] + face_plane_index(face, e, s[0], s[1], s[2])];
     else
-      return (T)face_value(g, a.f, a.t, c, face, s[0], s[1], s[2]);
+      return (T)face_value(
+          g, [&](int st, int cc, int pi, int pj, int pk) { return bc_eval<MODE>(g, a.f, a.t, a.tf, st, cc, pi, pj, pk); },
+          c, face, s[0], s[1], s[2]);
   }
   return F[L.idx(s[0], s[1], s[2])];
 }
@@ -879,7 +905,17 @@ __global__ void __launch_bounds__(256) k_div_rhs(DGrid g, Layout L, const T* __r
   const double dv_dy = ((double)v[o + L.PX] - (double)v[o]) * g.one_over_h[1];
   const double dw_dz = ((double)w[o + L.plane] - (double)w[o]) * g.one_over_h[2];
   double r = (du_dx + dv_dy + dw_dz) / dt;
-  if (NHN == 1) {
+  if (NHN == 3) {
+    // the Ethier-Steinman gradient from the axis tables, tg its time factor
+    // (65^3 nodes: 48 -> 6 us against the general evaluator)
+    const AxisEval at{gp.axis, gp.an, 3, {i, j, k}};
+    if (k == 0) r += at.es_grad_p(2, 0, 1) * tg * 2.0 * g.one_over_h[2];
+    if (k == g.N[2] - 1) r -= at.es_grad_p(2, 0, 1) * tg * 2.0 * g.one_over_h[2];
+    if (j == 0) r += at.es_grad_p(1, 2, 0) * tg * 2.0 * g.one_over_h[1];
+    if (j == g.N[1] - 1) r -= at.es_grad_p(1, 2, 0) * tg * 2.0 * g.one_over_h[1];
+    if (i == 0) r += at.es_grad_p(0, 1, 2) * tg * 2.0 * g.one_over_h[0];
+    if (i == g.N[0] - 1) r -= at.es_grad_p(0, 1, 2) * tg * 2.0 * g.one_over_h[0];
+  } else if (NHN == 1) {
     const int sx = g.N[0], sy = g.N[1], sz = g.N[2];
     if (k == 0) r += eval_at(g, gp, 3, 2, tg, i, j, k) * 2.0 * g.one_over_h[2];
     if (k == sz - 1) r -= eval_at(g, gp, 3, 2, tg, i, j, k) * 2.0 * g.one_over_h[2];
@@ -1265,7 +1301,7 @@ void launch_stage(int stage, const DGrid& g, const Layout& L, const StageArgs& s
 template <typename T>
 void launch_vel_stage(int stage, const DGrid& g, const Layout& L, const VelStageArgs& vs, hipStream_t st) {
   StageArgs s{};
-  const bool ft = vs.trig && vs.forcing.kind == MIF_FN_VT_FORCING;
+  const bool ft = vs.forcing.kind == MIF_FN_VT_FORCING;
   if (stage == 1)
     ft ? launch_stage_kind<T, 4, true>(g, L, s, vs, st) : launch_stage_kind<T, 4>(g, L, s, vs, st);
   else if (stage == 2)
@@ -1274,17 +1310,18 @@ void launch_vel_stage(int stage, const DGrid& g, const Layout& L, const VelStage
     ft ? launch_stage_kind<T, 6, true>(g, L, s, vs, st) : launch_stage_kind<T, 6>(g, L, s, vs, st);
 }
 
-__global__ void __launch_bounds__(256) k_trig_tables(DGrid g, double* __restrict__ trig, int tn) {
+__global__ void __launch_bounds__(256) k_axis_tables(DGrid g, double* __restrict__ tab, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const int a = blockIdx.y / 2, sh = blockIdx.y % 2;
-  if (i >= tn) return;
+  if (i >= n) return;
   const double x = coord(g, a, sh ? a : 3, i);
-  trig[((a * 2 + sh) * 2 + 0) * tn + i] = sin(x);
-  trig[((a * 2 + sh) * 2 + 1) * tn + i] = cos(x);
+  const double xa = MIF_PI / 4 * x, xd = MIF_PI / 2 * x;
+  const double v[kAxisFns] = {sin(x), cos(x), exp(xa), sin(xa), cos(xa), sin(xd), cos(xd)};
+  for (int f = 0; f < kAxisFns; f++) tab[axis_index(a, sh, f, n) + i] = v[f];
 }
 
-void launch_trig_tables(const DGrid& g, double* trig, int tn, hipStream_t st) {
-  k_trig_tables<<<dim3((tn + 255) / 256, 6, 1), 256, 0, st>>>(g, trig, tn);
+void launch_axis_tables(const DGrid& g, double* tab, int n, hipStream_t st) {
+  k_axis_tables<<<dim3((n + 255) / 256, 6, 1), 256, 0, st>>>(g, tab, n);
 }
 
 static void shell_counts(const DGrid& g, int stag, int cnt[3]) {
@@ -1312,26 +1349,29 @@ void launch_bc(const DGrid& g, const Layout& L, void* const F[3], const FnDesc& 
   a.f = f;
   a.t = t;
   const RimShape rs = rim_shape(g);
+  unsigned nbx = (unsigned)((mx + 255) / 256);
   if (rim.pin) {
     // three more block rows for the pressure rim, as many blocks as either needs
     const long rmx = max(rs.count[0], max(rs.count[1], rs.count[2]));
-    const unsigned nbx = (unsigned)max((long)(mx + 255) / 256, (rmx + 255) / 256);
-    const dim3 grd(nbx, 12, 1);
-    if (f.kind == MIF_FN_ZERO)
-      k_bc<T, BC_ZERO, true><<<grd, 256, 0, st>>>(g, L, a, rim, rs);
-    else if (f.kind == kFnFaceTable)
-      k_bc<T, BC_TABLE, true><<<grd, 256, 0, st>>>(g, L, a, rim, rs);
-    else
-      k_bc<T, BC_FN, true><<<grd, 256, 0, st>>>(g, L, a, rim, rs);
-    return;
+    nbx = (unsigned)max((long)nbx, (rmx + 255) / 256);
   }
-  dim3 grd((mx + 255) / 256, 9, 1);
-  if (f.kind == MIF_FN_ZERO)
-    k_bc<T, BC_ZERO><<<grd, 256, 0, st>>>(g, L, a, rim, rs);
-  else if (f.kind == kFnFaceTable)
-    k_bc<T, BC_TABLE><<<grd, 256, 0, st>>>(g, L, a, rim, rs);
-  else
-    k_bc<T, BC_FN><<<grd, 256, 0, st>>>(g, L, a, rim, rs);
+  auto go = [&](auto mode) {
+    constexpr int M = decltype(mode)::value;
+    if (M == BC_ES || M == BC_VT) a.tf = time_factor(f.kind, t, f.Re);
+    if (rim.pin)
+      k_bc<T, M, true><<<dim3(nbx, 12, 1), 256, 0, st>>>(g, L, a, rim, rs);
+    else
+      k_bc<T, M><<<dim3(nbx, 9, 1), 256, 0, st>>>(g, L, a, rim, rs);
+  };
+  switch (f.kind) {
+    case MIF_FN_ZERO: return go(std::integral_constant<int, BC_ZERO>{});
+    case kFnFaceTable: return go(std::integral_constant<int, BC_TABLE>{});
+    case MIF_FN_ES_VELOCITY: return go(std::integral_constant<int, BC_ES>{});
+    case MIF_FN_VT_VELOCITY: return go(std::integral_constant<int, BC_VT>{});
+    case MIF_FN_LID_1:
+    case MIF_FN_LID_2: return go(std::integral_constant<int, BC_LID>{});
+    default: return go(std::integral_constant<int, BC_FN>{});
+  }
 }
 
 template <typename T>
@@ -1359,6 +1399,11 @@ void launch_div_rhs(const DGrid& g, const Layout& L, const T* u, const T* v, con
   dim3 grd((g.npts[0] + 255) / 256, g.npts[1], g.npts[2]);
   if (nhn && gp.kind == kFnFaceTable)
     k_div_rhs<T, S, 2><<<grd, 256, 0, st>>>(g, L, u, v, w, B, bp0, bplane, dt, gp, tg);
+  else if (nhn && gp.kind == MIF_FN_ES_GRAD_P)
+    k_div_rhs<T, S, 3><<<grd, 256, 0, st>>>(g, L, u, v, w, B, bp0, bplane, dt, gp, time_factor(gp.kind, tg, gp.Re));
+  else if (nhn && gp.kind == MIF_FN_TIME_DIFFERENCE && gp.base == MIF_FN_ES_GRAD_P)
+    k_div_rhs<T, S, 3><<<grd, 256, 0, st>>>(g, L, u, v, w, B, bp0, bplane, dt, gp,
+                                            grad_p_factor_difference(gp.t1, gp.t0, gp.Re));
   else if (nhn)
     k_div_rhs<T, S, 1><<<grd, 256, 0, st>>>(g, L, u, v, w, B, bp0, bplane, dt, gp, tg);
   else
