@@ -1016,9 +1016,11 @@ int upload_face_tables(mif_ctx* c, bool velocity, const double* host, int count,
   return MIF_OK;
 }
 
-// Whether an axis has no specialised transform kernel.
+// Whether an axis needs the transform's matrices: no specialised kernel, or an
+// x axis short enough for dense_x_short.
 bool dense_axis(int axis, const FftPlan& P) {
-  if (P.dct2 || P.L < 2 || fft_fast_len(P.L)) return false;
+  if (P.dct2 || P.L < 2) return false;
+  if (fft_fast_len(P.L)) return axis == 0 && P.L <= 128;
   // the half-length DCT-I of long wall-normal y axes
   return !(axis == 1 && !P.periodic && (P.L == 1024 || P.L == 1536 || P.L == 2048));
 }
@@ -1149,13 +1151,15 @@ int ctx_init(mif_ctx* c, const mif_grid* grid, const uint64_t Ng[3], int precisi
       add_table(&P.H64, h64);
       add_table(&P.H32, h32);
     }
-    if (dense_axis(a, P) && dense_plan(n, P.periodic, &P.dense)) {
+    const bool dense = dense_axis(a, P) && dense_plan(n, P.periodic, &P.dense);
+    if (dense) {
       std::vector<double> m64(dense_table_elems(P.dense));
       std::vector<float> m32(f32 ? m64.size() : 0);
       dense_table(P.dense, m64.data(), f32 ? m32.data() : nullptr);
       add_table(&P.dense.M64, m64);
       add_table(&P.dense.M32, m32);
-    } else {
+    }
+    if (!dense || fft_fast_len(P.L)) {
       std::vector<double> w64(2 * (size_t)P.L);
       std::vector<float> w32(f32 ? 2 * (size_t)P.L : 0);
       for (int e = 0; e < P.L; e++) {

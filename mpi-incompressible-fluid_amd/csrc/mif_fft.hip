@@ -392,7 +392,8 @@ void launch_fft_axis(const DGrid& g, int axis, int dir, int fused, const FftPlan
     (void)launch_dct2_y_any<T>(g, plan, dir > 0, B, bp0, bplane, st);
     return;
   }
-  if (plan.L >= 2 && launch_fft_pow2<T>(g, axis, mode, plan, sc, B, bp0, bplane, nullptr, st)) return;
+  const bool dense_first = axis == 0 && dense_x_short(g, plan, sizeof(T) == 8);
+  if (!dense_first && plan.L >= 2 && launch_fft_pow2<T>(g, axis, mode, plan, sc, B, bp0, bplane, nullptr, st)) return;
   if (plan.dense.M64) {
     launch_dense<T>(g, axis, mode, plan.dense, sc, B, bp0, bplane, nullptr, st);
     return;
@@ -408,12 +409,34 @@ void launch_fft_axis(const DGrid& g, int axis, int dir, int fused, const FftPlan
   }
 }
 
+// Short x lines that have a specialised kernel but run as matrix products:
+// that kernel holds 16 to 32 lines per workgroup there, and neither its
+// workgroups nor its threads fill the device while there are few lines.
+// Divergence / unpack pass, specialised -> products (us): FP64 64 periodic
+// points on 65^2 lines 13.4 / 15.2 -> 10.6 / 10.2, 129^2 16.6 / 17.2 -> 16.1 /
+// 13.8, 257^2 31.7 / 26.7 -> 40.8 / 30.4 (so not there); 33 and 49 wall nodes
+// at every line count, 257^2: 29.4 / 27.6 -> 25.2 / 20.1 and 44.0 / 24.5 -> 28.3
+// / 21.1; FP32 96 points on 129^2 17.5 / 16.7 -> 14.0 / 12.8; FP64 128 points
+// on 129^2 19.9 / 14.8 -> 24.5 / 19.1 (so FP64 lines of more than 65 points keep
+// theirs).
+bool dense_x_short(const DGrid& g, const FftPlan& plan, bool fp64) {
+  if (!plan.dense.M64 || plan.L > 128 || !fft_fast_len(plan.L)) return false;
+  if (!plan.periodic && plan.L <= 96) return true;
+  return !(fp64 && plan.n > 65) && pow2_x_blocks(g, plan, fp64) < 1500;
+}
+
 bool fused_x_pass(const FftPlan& plan) { return fft_fast_len(plan.L) || plan.dense.M64; }
+
+int fused_x_blocks(const DGrid& g, const FftPlan& plan, bool fp64) {
+  if (fft_fast_len(plan.L) && !dense_x_short(g, plan, fp64)) return pow2_x_blocks(g, plan, fp64);
+  return plan.dense.M64 ? dense_x_blocks(g) : 0;
+}
 
 template <typename T>
 void launch_fused_x(const DGrid& g, int mode, const FftPlan& plan, const SpectralScale& sc, T* B, long bp0, long bplane,
                     const FusedIO& io, hipStream_t st) {
-  if (launch_fft_pow2<T>(g, 0, mode, plan, sc, B, bp0, bplane, &io, st)) return;
+  if (!dense_x_short(g, plan, sizeof(T) == 8) && launch_fft_pow2<T>(g, 0, mode, plan, sc, B, bp0, bplane, &io, st))
+    return;
   launch_dense<T>(g, 0, mode, plan.dense, sc, B, bp0, bplane, &io, st);
 }
 

@@ -1170,7 +1170,7 @@ bool launch_fft_pow2(const DGrid& g, int axis, int mode, const FftPlan& plan, co
 
 // Workgroups of the x pass launch_fft_pow2 runs for a plan (its line pairs
 // per workgroup follow the same table); 0 when the length has no kernel.
-int fused_x_blocks(const DGrid& g, const FftPlan& plan, bool fp64) {
+int pow2_x_blocks(const DGrid& g, const FftPlan& plan, bool fp64) {
   int np;
   switch (plan.L) {
     case 64: np = np_strided(fp64, 64); break;
@@ -1182,7 +1182,7 @@ int fused_x_blocks(const DGrid& g, const FftPlan& plan, bool fp64) {
     case 384: np = np_x(fp64, 384); break;
     case 768: np = np_x(fp64, 768); break;
     case 1024: case 1536: np = 1; break;
-    default: return plan.dense.M64 ? dense_x_blocks(g) : 0;
+    default: return 0;
   }
   const long lines = (long)g.npts[1] * g.npts[2];
   return (int)((lines + 2 * np - 1) / (2 * np));

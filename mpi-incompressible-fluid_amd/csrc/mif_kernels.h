@@ -227,8 +227,10 @@ bool fused_x_pass(const FftPlan& plan);
 template <typename T>
 void launch_fused_x(const DGrid& g, int mode, const FftPlan& plan, const SpectralScale& sc, T* B, long bp0, long bplane,
                     const FusedIO& io, hipStream_t st);
-// Workgroups of the specialised x pass of a plan (0 without a kernel): the
-// number of partial sums a fused x pass with FusedIO::dc leaves.
+bool dense_x_short(const DGrid& g, const FftPlan& plan, bool fp64);
+// Workgroups of the specialised x pass of a plan (0 without one), and of the
+// fused x pass that runs: the number of partial sums FusedIO::dc leaves.
+int pow2_x_blocks(const DGrid& g, const FftPlan& plan, bool fp64);
 int fused_x_blocks(const DGrid& g, const FftPlan& plan, bool fp64);
 // DCT-II (forward) or DCT-III (inverse) pass of a cell-centred Neumann y
 // axis; false when the length (64, 128, 256, 512 or 1024) has no kernel.

@@ -59,7 +59,10 @@ def test_poisson_solve_per_axis(axis, n, per):
 
 
 FUSED = [((32, 18, 20), (0, 0, 0)), ((33, 18, 21), (1, 0, 1)), ((102, 21, 19), (1, 1, 1)), ((287, 9, 14), (0, 1, 0)),
-         ((7, 40, 33), (1, 0, 1))]
+         ((7, 40, 33), (1, 0, 1)),
+         # short x lines with a specialised kernel that run as products
+         ((33, 20, 18), (0, 0, 0)), ((65, 20, 18), (1, 0, 1)), ((65, 18, 9), (0, 1, 1)), ((97, 12, 14), (1, 0, 1)),
+         ((129, 12, 14), (1, 0, 0))]
 
 
 @pytest.mark.parametrize("Ng,per", FUSED, ids=lambda v: "x".join(map(str, v)))
