@@ -227,6 +227,7 @@ struct AxisEval {
   }
   // es_u, es_dpdx with (x, y, z) = axes (p, q, r)
   __device__ inline double es_velocity(int p, int q, int r) const {
+#pragma clang fp contract(off)
     return -(MIF_PI / 4) * ((*this)(p, AX_EXP_A) * sin_ad(q, r) + (*this)(r, AX_EXP_A) * cos_ad(p, q));
   }
   __device__ inline double es_grad_p(int p, int q, int r) const {
@@ -239,6 +240,7 @@ struct AxisEval {
     return -a * a / 2 * v;
   }
   __device__ inline double vt_velocity(int c) const {
+#pragma clang fp contract(off)
     if (c == 0) return (*this)(0, AX_SIN) * (*this)(1, AX_COS) * (*this)(2, AX_SIN);
     if (c == 1) return (*this)(0, AX_COS) * (*this)(1, AX_SIN) * (*this)(2, AX_SIN);
     return 2 * (*this)(0, AX_COS) * (*this)(1, AX_COS) * (*this)(2, AX_COS);

@@ -718,6 +718,9 @@ enum BCMode { BC_ZERO = 0, BC_FN = 1, BC_TABLE = 2, BC_ES = 3, BC_VT = 4, BC_LID
 template <int MODE>
 __device__ inline double bc_eval(const DGrid& g, const FnDesc& f, double t, double tf, int s, int c, int i, int j,
                                  int k) {
+// a value is rounded before the differences of face_value take it, so that
+// equal points give equal values whichever product would be fused
+#pragma clang fp contract(off)
   if constexpr (MODE == BC_ES || MODE == BC_VT) {
     const AxisEval at{f.axis, f.an, s, {i, j, k}};
     if constexpr (MODE == BC_VT) return at.vt_velocity(c) * tf;
