@@ -24,6 +24,8 @@
 // z_bar and N_bar vanish outside the component interiors (the forward
 // computes N and writes the stage update only there), which lets k_adj_xb
 // read neighbours without interior tests.
+#include <algorithm>
+
 #include "mif_kernels.h"
 
 namespace mif {
@@ -64,14 +66,27 @@ __device__ inline int images(const DGrid& g, int a, int P, int s, int out[2]) {
 //   phi_bar(R) = p_bar(R) + dt_s sum_c (y_bar_c(R + e_c) - y_bar_c(R)) / h_c
 // with y_bar_c taken on the interior of component c only.
 // ---------------------------------------------------------------------------
+// A wave takes 64 points of a row at a time, so that the row's tests and
+// addresses are uniform and the loads contiguous (128^3 FP64 right-hand side:
+// 38.5 -> 32.8 us against one point per thread with its own index division).
+struct RowItem {
+  int i, j, k;
+};
+// Item w of rows of n0 points, n1 rows per plane: nx = ceil(n0 / 64) items per row.
+__device__ inline RowItem row_item(int w, int nx, int n1) {
+  const int row = w / nx, iw = w - row * nx;
+  const int k = row / n1;
+  return {64 * iw + (int)(threadIdx.x & 63), row - k * n1, k};
+}
+
 template <typename T>
 __global__ void __launch_bounds__(256) k_adj_rhs(DGrid g, Layout L, const T* __restrict__ P, AdjVec Y, double dts,
-                                                 T* __restrict__ B, long bp0, long bplane, long total) {
-  // flat indices fit in 32 bits (the context bounds every field below 2^31
-  // elements), so the decomposition uses 32-bit division
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= total) return;
-  const int a = q % g.npts[0], rq = q / g.npts[0], b = rq % g.npts[1], c = rq / g.npts[1];
+                                                 T* __restrict__ B, long bp0, long bplane, int nx, int items) {
+  const int w0 = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+  if (w0 >= items) return;
+  const RowItem q = row_item(w0, nx, g.npts[1]);
+  const int a = q.i, b = q.j, c = q.k;
+  if (a >= g.npts[0]) return;
   const int O[3] = {a + g.olo[0], b + g.olo[1], c + g.olo[2]};
   const long off[3] = {1, L.PX, L.plane};
   // R and R + e_c lie inside the padded array for every pressure point R,
@@ -100,47 +115,44 @@ __global__ void __launch_bounds__(256) k_adj_rhs(DGrid g, Layout L, const T* __r
     }
     return pv + dts * acc;
   };
+  double s = phib(O[0], O[1], O[2]);
   int opts[3][2], nopt[3];
   bool single = true;
   for (int ax = 0; ax < 3; ax++) {
     nopt[ax] = images(g, ax, O[ax], g.N[ax], opts[ax]);
     single = single && nopt[ax] == 1;
   }
-  double s = 0;
-  if (single) {
-    s = phib(O[0], O[1], O[2]);
-  } else {
+  if (!single) {
     for (int qa = 0; qa < nopt[0]; qa++)
       for (int qb = 0; qb < nopt[1]; qb++)
-        for (int qc = 0; qc < nopt[2]; qc++) s += phib(opts[0][qa], opts[1][qb], opts[2][qc]);
+        for (int qc = 0; qc < nopt[2]; qc++)
+          if (qa + qb + qc > 0) s += phib(opts[0][qa], opts[1][qb], opts[2][qc]);
   }
+  // (the weight is a power of two: its reciprocal is exact)
   const double w = trap_weight(g, 0, a) * trap_weight(g, 1, b) * trap_weight(g, 2, c);
-  B[a + bp0 * b + bplane * c] = (T)(s / w);
+  B[a + bp0 * b + bplane * c] = (T)(w == 1.0 ? s : s * (w == 0.5 ? 2.0 : (w == 0.25 ? 4.0 : 8.0)));
 }
 
 // ---------------------------------------------------------------------------
-// k_adj_zb: component c = blockIdx.y, interior points Q of c (grid-stride):
+// k_adj_zb: interior points Q of the three components c,
 //   z_bar_c(Q) = sum over the points g holding Q (Q and its periodic ghost
 //                copies) of y_bar_c(g) + (Wpsi(g - e_c) - Wpsi(g)) / (dt_s h_c)
 //   N_bar_c(Q) = alpha z_bar_c(Q) + beta Zo_c(Q)
 // with Wpsi = W * psi on owner nodes (zero elsewhere), and per workgroup the
-// partial sum of z_bar_c weighted by fcoef, stored (accumulate = 0) or added
+// partial sums of z_bar_c weighted by fcoef, stored (accumulate = 0) or added
 // to the workgroup's slot (accumulate = 1: the later stages of one adjoint
 // step, launched with the same grid, so slot b always belongs to workgroup b).
+// Waves take 64 points of a row at a time (row_item), all components together,
+// so that psi is read once for the three; hd holds 1 / (dt_s h_c).  128^3 FP64:
+// 91 -> 62 us against one component and point per thread (10 to 13 words per
+// point at about 3 TB/s).
 // ---------------------------------------------------------------------------
 template <typename T>
 __global__ void __launch_bounds__(256) k_adj_zb(DGrid g, Layout L, AdjVec Y, const T* __restrict__ Bpsi, long bp0,
-                                                long bplane, double dts, AdjVec Zb, AdjVec Nb, AdjVec Zo, double alpha,
-                                                double beta, double fcoef, int accumulate, double* __restrict__ partial) {
-  const int c = blockIdx.y;
-  int e[3];
-  extents(g, c, e);
-  const int n0 = e[0] - 2, n1 = e[1] - 2, n2 = e[2] - 2;
-  const int total = (n0 > 0 && n1 > 0 && n2 > 0) ? n0 * n1 * n2 : 0;
-  const T* y = (const T*)Y.f[c];
-  T* zb = (T*)Zb.f[c];
-  T* nb = (T*)Nb.f[c];
-  const T* zo = (const T*)Zo.f[c];
+                                                long bplane, double hd0, double hd1, double hd2, AdjVec Zb, AdjVec Nb,
+                                                AdjVec Zo, double alpha, double beta, double fcoef, int accumulate,
+                                                double* __restrict__ partial, int jmax, int nx, int items) {
+  const double hd[3] = {hd0, hd1, hd2};
   // W * psi at pressure point P (zero off the owner nodes); the load reads
   // a valid address either way
   auto wpsi = [&](int pi, int pj, int pk) -> double {
@@ -151,46 +163,64 @@ __global__ void __launch_bounds__(256) k_adj_zb(DGrid g, Layout L, AdjVec Y, con
     const double w = trap_weight(g, 0, q0) * trap_weight(g, 1, q1) * trap_weight(g, 2, q2);
     return ok ? w * v : 0.0;
   };
-  double part = 0;
-  for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < total; q += gridDim.x * blockDim.x) {
-    const int rq = q / n0;
-    const int Q[3] = {q % n0 + 1, rq % n1 + 1, rq / n1 + 1};
-    auto term = [&](int g0, int g1, int g2) -> double {
-      int Gm[3] = {g0, g1, g2};
-      Gm[c] -= 1;
-      const double d = (wpsi(Gm[0], Gm[1], Gm[2]) - wpsi(g0, g1, g2)) * g.one_over_h[c] / dts;
-      return (double)(T)((double)y[L.idx(g0, g1, g2)] + d);
-    };
-    int opts[3][2], nopt[3];
-    bool single = true;
-    for (int ax = 0; ax < 3; ax++) {
-      nopt[ax] = images(g, ax, Q[ax], e[ax], opts[ax]);
-      single = single && nopt[ax] == 1;
-    }
-    double s = 0;
-    if (single) {
-      s = term(Q[0], Q[1], Q[2]);
-    } else {
-      for (int qa = 0; qa < nopt[0]; qa++)
-        for (int qb = 0; qb < nopt[1]; qb++)
-          for (int qc = 0; qc < nopt[2]; qc++) s += term(opts[0][qa], opts[1][qb], opts[2][qc]);
-    }
-    const long o = L.idx(Q[0], Q[1], Q[2]);
-    const T z = (T)s;
-    zb[o] = z;
+  double part[3] = {0, 0, 0};
+  const int nw = gridDim.x * 4;
+  for (int it = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6)); it < items; it += nw) {
+    const RowItem r = row_item(it, nx, jmax);
+    const int i = r.i + 1, j = r.j + 1, k = r.k + 1;
+    const long o = L.idx(min(i, L.PX - 1), j, k);
+    const double here = wpsi(i, j, k);
+    const double below[3] = {wpsi(i - 1, j, k), wpsi(i, j - 1, k), wpsi(i, j, k - 1)};
+    T y[3], zo[3] = {(T)0, (T)0, (T)0};
+#pragma unroll
+    for (int c = 0; c < 3; c++) y[c] = ((const T*)Y.f[c])[o];
     // the later stage's z_bar enters only with beta != 0 (stage 2): the
     // other stages skip its load (a uniform branch)
-    double nbv = alpha * (double)z;
-    if (beta != 0.0) nbv += beta * (double)zo[o];
-    nb[o] = (T)nbv;
-    part += (double)z;
+    if (beta != 0.0) {
+#pragma unroll
+      for (int c = 0; c < 3; c++) zo[c] = ((const T*)Zo.f[c])[o];
+    }
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      int e[3];
+      extents(g, c, e);
+      if (i > e[0] - 2 || j > e[1] - 2 || k > e[2] - 2) continue;
+      double s = (double)(T)((double)y[c] + (below[c] - here) * hd[c]);
+      int opts[3][2], nopt[3];
+      const int Q[3] = {i, j, k};
+      bool single = true;
+      for (int ax = 0; ax < 3; ax++) {
+        nopt[ax] = images(g, ax, Q[ax], e[ax], opts[ax]);
+        single = single && nopt[ax] == 1;
+      }
+      if (!single) {
+        for (int qa = 0; qa < nopt[0]; qa++)
+          for (int qb = 0; qb < nopt[1]; qb++)
+            for (int qc = 0; qc < nopt[2]; qc++) {
+              if (qa + qb + qc == 0) continue;
+              const int g0 = opts[0][qa], g1 = opts[1][qb], g2 = opts[2][qc];
+              const double d = (wpsi(g0 - (c == 0), g1 - (c == 1), g2 - (c == 2)) - wpsi(g0, g1, g2)) * hd[c];
+              s += (double)(T)((double)((const T*)Y.f[c])[L.idx(g0, g1, g2)] + d);
+            }
+      }
+      const T z = (T)s;
+      ((T*)Zb.f[c])[o] = z;
+      double nbv = alpha * (double)z;
+      if (beta != 0.0) nbv += beta * (double)zo[c];
+      ((T*)Nb.f[c])[o] = (T)nbv;
+      part[c] += (double)z;
+    }
   }
-  __shared__ double sh[4];
-  for (int off = 32; off > 0; off >>= 1) part += __shfl_down(part, off, 64);
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = part;
+  __shared__ double sh[3][4];
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    for (int off = 32; off > 0; off >>= 1) part[c] += __shfl_down(part[c], off, 64);
+    if ((threadIdx.x & 63) == 0) sh[c][threadIdx.x >> 6] = part[c];
+  }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    const double v = fcoef * (sh[0] + sh[1] + sh[2] + sh[3]);
+  if (threadIdx.x < 3) {
+    const int c = threadIdx.x;
+    const double v = fcoef * (sh[c][0] + sh[c][1] + sh[c][2] + sh[c][3]);
     double* slot = &partial[c * gridDim.x + blockIdx.x];
     *slot = accumulate ? *slot + v : v;
   }
@@ -232,217 +262,246 @@ __global__ void __launch_bounds__(kAdjSumThreads) k_adj_sum(const double* __rest
 // k_adj_xb: for every point Q of the three components,
 //   x_bar_c(Q) = z_bar_c(Q) + (J_N(X)^T N_bar)_c(Q)
 // and, at pressure points, p_bar(Q) += b sum_c (z_bar_c(Q + e_c) - z_bar_c(Q)) / h_c.
-// N_bar and z_bar are zero outside the component interiors and in the
-// padding, and every tap index is clamped into the array, so taps need no
-// tests: a clamped N_bar tap reads a boundary or padding cell (zero) and the
-// X value it multiplies is finite.
+//
+// With n = N_bar and (a, b) ranging over the axes, N's component c at P holds
+// -x_c D_c x_c - sum_a (S_a^c) D_a x_c with S_a^c the four-point sum of x_a
+// around P; its transpose needs, per point P, the products
+//   G_c(P)   = n_c x_c
+//   H_c^a(P) = n_c S_a^c,    S_a^c = x_a(P+a) + x_a(P) + x_a(P-c+a) + x_a(P-c)
+//   F_c^a(P) = n_c (x_c(P+a) - x_c(P-a))
+// and then, for component c at Q,
+//   x_bar_c = z_bar_c + diffusion(n_c) - n_c (x_c(Q+c) - x_c(Q-c)) / 2h_c
+//             + (G_c(Q+c) - G_c(Q-c)) / 2h_c + sum_a (H_c^a(Q+a) - H_c^a(Q-a)) / 8h_a
+//             - sum_a (F_a^c(Q) + F_a^c(Q-c) + F_a^c(Q+a) + F_a^c(Q+a-c)) / 8h_c
+// so that every product is formed once per point instead of at each of the
+// points that gather it (which takes X two points away).
+//
+// A workgroup's 32 x 16 threads are the points of a tile with a one-point
+// halo (30 x 14 outputs) and march along k.  The products of a plane go
+// through LDS; everything that couples planes stays in registers of the
+// column: the four-point sums' halves, the plane differences and the
+// contributions to the planes below and above.  X itself needs one plane in
+// LDS at a time, with one more halo point.  N_bar is zero outside the component
+// interiors and cells outside the arrays read as zero, so no product needs a
+// test.  76 KB of LDS, two workgroups (16 waves) per CU; the arithmetic is FP64
+// in both forms.  Bound by the LDS and the plane's two barriers: 128^3 FP64 153 ->
+// 99 us against gathering X and N_bar from a three-plane ring of six fields (8
+// waves per CU, 31 global taps per point); 14 words per point at 2.4 TB/s.  A
+// kernel that spills here is slower than that one (the reloads wait for every
+// load in flight): 128 VGPRs hold it only with one address register per load.
 // ---------------------------------------------------------------------------
-// x_bar at one point Q = (i, j, k) from tap providers: tp(f, di, dj, dk)
-// returns X_f (f = 0..2) or N_bar_{f-3} (f = 3..5) at Q + (di, dj, dk), and
-// zt(c, di, dj, dk) returns z_bar_c there.  Offsets are literals at every
-// call site, so a provider can pick its source at compile time.
-template <typename T, typename TP, typename ZT>
-__device__ inline void adj_xb_point(const DGrid& g, long o, int i, int j, int k, TP tp, ZT zt, T* __restrict__ XB0,
-                                    T* __restrict__ XB1, T* __restrict__ XB2, T* __restrict__ P, double bcoef) {
+constexpr int AXT = 32, AYT = 16;            // threads: the tile with its halo
+constexpr int AOX = AXT - 2, AOY = AYT - 2;  // outputs
+constexpr int AHX = AXT + 2, AHY = AYT + 2;  // X plane
+constexpr int ARING = 2 * (AHX + AYT);       // X plane points outside the threads' own
+enum AdjProduct { PN_U, PN_V, PN_W, PG_V, PH_UV, PH_VU, PH_WU, PH_WV, PF_UY, PF_VX, PF_VZ, PF_WY, kAdjProducts };
+
+template <typename T>
+__global__ void __launch_bounds__(AXT * AYT) __attribute__((amdgpu_waves_per_eu(4)))
+k_adj_xb(DGrid g, Layout L, AdjVec Xv, AdjVec Nbv, AdjVec Zv, AdjVec Xbv, T* __restrict__ P, double bcoef, int ntx,
+         int nty, int ntiles, int kchunk) {
+  __shared__ T xs[2][3][AHY][AHX];
+  __shared__ double pr[kAdjProducts][AYT][AXT];
+  const int tid = threadIdx.x, tx = tid % AXT, ty = tid / AXT;
+  const int tile = xcd_tile(blockIdx.x, ntiles);
+  const int bx = tile % ntx, by = (tile / ntx) % nty, bz = tile / (ntx * nty);
+  const int i = bx * AOX - 1 + tx, j = by * AOY - 1 + ty;
+  const int k0 = bz * kchunk, kend = min(k0 + kchunk, g.N[2] + 1);  // output planes k0 .. kend-1
+  const T* X[3] = {(const T*)Xv.f[0], (const T*)Xv.f[1], (const T*)Xv.f[2]};
+  const T* N[3] = {(const T*)Nbv.f[0], (const T*)Nbv.f[1], (const T*)Nbv.f[2]};
+  const T* Z[3] = {(const T*)Zv.f[0], (const T*)Zv.f[1], (const T*)Zv.f[2]};
+  // this thread's column, and its point of the X plane's outer ring
+  const bool own = i >= 0 && j >= 0 && i < L.PX && j < L.SY;
+  // lane offsets are 32-bit and the plane's base is uniform, so that a load
+  // takes one address register
+  const unsigned oo = own ? i + L.PX * j : 0;
+  int rx = 0, ry = 0;
+  if (tid < AHX) {
+    rx = tid;
+  } else if (tid < 2 * AHX) {
+    rx = tid - AHX;
+    ry = AHY - 1;
+  } else if (tid < ARING) {
+    rx = (tid - 2 * AHX) < AYT ? 0 : AHX - 1;
+    ry = 1 + (tid - 2 * AHX) % AYT;
+  }
+  const int ri = bx * AOX - 2 + rx, rj = by * AOY - 2 + ry;
+  const bool ring = tid < ARING;
+  const bool rok = ring && ri >= 0 && rj >= 0 && ri < L.PX && rj < L.SY;
+  const unsigned ro = rok ? ri + L.PX * rj : 0;
+
+  // planes outside the arrays read plane 0 and count as zero
+  auto plane_ok = [&](int k) { return k >= 0 && k < L.SZ; };
+  auto plane_at = [&](int k) -> long { return plane_ok(k) ? (long)k * L.plane : 0; };
+  // (kept out of the compiler's sight from plane to plane: hoisted out of the
+  // loop, the sums of base and offset take a register pair per array)
+  auto lane = [](unsigned off) {
+    asm volatile("" : "+v"(off));
+    return off;
+  };
+  T px[3], pring[3], pn[3];
+  auto fetch_x = [&](int k) {
+    const long kp = plane_at(k);
+    const unsigned a = lane(oo), b = lane(ro);
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      const T* x = X[c] + kp;
+      px[c] = x[a];
+      pring[c] = x[b];
+    }
+  };
+  auto fetch_n = [&](int k) {
+    const long kp = plane_at(k);
+    const unsigned a = lane(oo);
+#pragma unroll
+    for (int c = 0; c < 3; c++) pn[c] = (N[c] + kp)[a];
+  };
+  auto commit_x = [&](int k) {
+    const bool kin = plane_ok(k);
+    T(&pl)[3][AHY][AHX] = xs[k & 1];
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      pl[c][ty + 1][tx + 1] = own && kin ? px[c] : (T)0;
+      if (ring) pl[c][ry][rx] = rok && kin ? pring[c] : (T)0;
+    }
+  };
+
   const double A2 = g.one_over_2h[0], B2 = g.one_over_2h[1], C2 = g.one_over_2h[2];
   const double A8 = g.one_over_8h[0], B8 = g.one_over_8h[1], C8 = g.one_over_8h[2];
   const double Dx = g.one_over_h2Re[0], Dy = g.one_over_h2Re[1], Dz = g.one_over_h2Re[2];
-  const double Dsum = Dx + Dy + Dz;
+  const double D2 = 2 * (Dx + Dy + Dz);
+  const bool out = tx >= 1 && ty >= 1 && tx <= AOX && ty <= AOY && i <= g.N[0] && j <= g.N[1];
+  // the column of a pressure point (its neighbours above lie in the arrays)
+  const bool pcol = out && i < g.N[0] && j < g.N[1];
+  const unsigned oz = pcol ? oo : 0;
 
-  // u at Q
-  if (in_field(g, 0, i, j, k)) {
-    double acc = zt(0, 0, 0, 0);
-    acc += tp(3, 0, 0, 0) * (-(tp(0, 1, 0, 0) - tp(0, -1, 0, 0)) * A2 - 2 * Dsum);
-    acc += tp(3, -1, 0, 0) * (-tp(0, -1, 0, 0) * A2 + Dx);
-    acc += tp(3, 1, 0, 0) * (tp(0, 1, 0, 0) * A2 + Dx);
-    // Vs_u(P) = v(P+y) + v(P) + v(P-x+y) + v(P-x), at P = Q -+ y
-    const double vsm = tp(1, 0, 0, 0) + tp(1, 0, -1, 0) + tp(1, -1, 0, 0) + tp(1, -1, -1, 0);
-    const double vsp = tp(1, 0, 2, 0) + tp(1, 0, 1, 0) + tp(1, -1, 2, 0) + tp(1, -1, 1, 0);
-    acc += tp(3, 0, -1, 0) * (-vsm * B8 + Dy);
-    acc += tp(3, 0, 1, 0) * (vsp * B8 + Dy);
-    // Ws_u(P) = w(P+z) + w(P) + w(P-x+z) + w(P-x), at P = Q -+ z
-    const double wsm = tp(2, 0, 0, 0) + tp(2, 0, 0, -1) + tp(2, -1, 0, 0) + tp(2, -1, 0, -1);
-    const double wsp = tp(2, 0, 0, 2) + tp(2, 0, 0, 1) + tp(2, -1, 0, 2) + tp(2, -1, 0, 1);
-    acc += tp(3, 0, 0, -1) * (-wsm * C8 + Dz);
-    acc += tp(3, 0, 0, 1) * (wsp * C8 + Dz);
-    // from the v equation at P = Q-x, Q, Q-x+y, Q+y: -(v(P+x) - v(P-x)) A8
-    acc += tp(4, -1, 0, 0) * (-(tp(1, 0, 0, 0) - tp(1, -2, 0, 0)) * A8);
-    acc += tp(4, 0, 0, 0) * (-(tp(1, 1, 0, 0) - tp(1, -1, 0, 0)) * A8);
-    acc += tp(4, -1, 1, 0) * (-(tp(1, 0, 1, 0) - tp(1, -2, 1, 0)) * A8);
-    acc += tp(4, 0, 1, 0) * (-(tp(1, 1, 1, 0) - tp(1, -1, 1, 0)) * A8);
-    // from the w equation at P = Q-x, Q, Q-x+z, Q+z: -(w(P+x) - w(P-x)) A8
-    acc += tp(5, -1, 0, 0) * (-(tp(2, 0, 0, 0) - tp(2, -2, 0, 0)) * A8);
-    acc += tp(5, 0, 0, 0) * (-(tp(2, 1, 0, 0) - tp(2, -1, 0, 0)) * A8);
-    acc += tp(5, -1, 0, 1) * (-(tp(2, 0, 0, 1) - tp(2, -2, 0, 1)) * A8);
-    acc += tp(5, 0, 0, 1) * (-(tp(2, 1, 0, 1) - tp(2, -1, 0, 1)) * A8);
-    XB0[o] = (T)acc;
-  }
-  // v at Q
-  if (in_field(g, 1, i, j, k)) {
-    double acc = zt(1, 0, 0, 0);
-    // from the u equation at P = Q-y, Q, Q+x-y, Q+x: -(u(P+y) - u(P-y)) B8
-    acc += tp(3, 0, -1, 0) * (-(tp(0, 0, 0, 0) - tp(0, 0, -2, 0)) * B8);
-    acc += tp(3, 0, 0, 0) * (-(tp(0, 0, 1, 0) - tp(0, 0, -1, 0)) * B8);
-    acc += tp(3, 1, -1, 0) * (-(tp(0, 1, 0, 0) - tp(0, 1, -2, 0)) * B8);
-    acc += tp(3, 1, 0, 0) * (-(tp(0, 1, 1, 0) - tp(0, 1, -1, 0)) * B8);
-    acc += tp(4, 0, 0, 0) * (-(tp(1, 0, 1, 0) - tp(1, 0, -1, 0)) * B2 - 2 * Dsum);
-    // Us_v(P) = u(P+x) + u(P) + u(P+x-y) + u(P-y), at P = Q -+ x
-    const double usm = tp(0, 0, 0, 0) + tp(0, -1, 0, 0) + tp(0, 0, -1, 0) + tp(0, -1, -1, 0);
-    const double usp = tp(0, 2, 0, 0) + tp(0, 1, 0, 0) + tp(0, 2, -1, 0) + tp(0, 1, -1, 0);
-    acc += tp(4, -1, 0, 0) * (-usm * A8 + Dx);
-    acc += tp(4, 1, 0, 0) * (usp * A8 + Dx);
-    acc += tp(4, 0, -1, 0) * (-tp(1, 0, -1, 0) * B2 + Dy);
-    acc += tp(4, 0, 1, 0) * (tp(1, 0, 1, 0) * B2 + Dy);
-    // Ws_v(P) = w(P+z) + w(P) + w(P-y+z) + w(P-y), at P = Q -+ z
-    const double wsm = tp(2, 0, 0, 0) + tp(2, 0, 0, -1) + tp(2, 0, -1, 0) + tp(2, 0, -1, -1);
-    const double wsp = tp(2, 0, 0, 2) + tp(2, 0, 0, 1) + tp(2, 0, -1, 2) + tp(2, 0, -1, 1);
-    acc += tp(4, 0, 0, -1) * (-wsm * C8 + Dz);
-    acc += tp(4, 0, 0, 1) * (wsp * C8 + Dz);
-    // from the w equation at P = Q-y, Q, Q-y+z, Q+z: -(w(P+y) - w(P-y)) B8
-    acc += tp(5, 0, -1, 0) * (-(tp(2, 0, 0, 0) - tp(2, 0, -2, 0)) * B8);
-    acc += tp(5, 0, 0, 0) * (-(tp(2, 0, 1, 0) - tp(2, 0, -1, 0)) * B8);
-    acc += tp(5, 0, -1, 1) * (-(tp(2, 0, 0, 1) - tp(2, 0, -2, 1)) * B8);
-    acc += tp(5, 0, 0, 1) * (-(tp(2, 0, 1, 1) - tp(2, 0, -1, 1)) * B8);
-    XB1[o] = (T)acc;
-  }
-  // w at Q
-  if (in_field(g, 2, i, j, k)) {
-    double acc = zt(2, 0, 0, 0);
-    // from the u equation at P = Q-z, Q, Q+x-z, Q+x: -(u(P+z) - u(P-z)) C8
-    acc += tp(3, 0, 0, -1) * (-(tp(0, 0, 0, 0) - tp(0, 0, 0, -2)) * C8);
-    acc += tp(3, 0, 0, 0) * (-(tp(0, 0, 0, 1) - tp(0, 0, 0, -1)) * C8);
-    acc += tp(3, 1, 0, -1) * (-(tp(0, 1, 0, 0) - tp(0, 1, 0, -2)) * C8);
-    acc += tp(3, 1, 0, 0) * (-(tp(0, 1, 0, 1) - tp(0, 1, 0, -1)) * C8);
-    // from the v equation at P = Q-z, Q, Q+y-z, Q+y: -(v(P+z) - v(P-z)) C8
-    acc += tp(4, 0, 0, -1) * (-(tp(1, 0, 0, 0) - tp(1, 0, 0, -2)) * C8);
-    acc += tp(4, 0, 0, 0) * (-(tp(1, 0, 0, 1) - tp(1, 0, 0, -1)) * C8);
-    acc += tp(4, 0, 1, -1) * (-(tp(1, 0, 1, 0) - tp(1, 0, 1, -2)) * C8);
-    acc += tp(4, 0, 1, 0) * (-(tp(1, 0, 1, 1) - tp(1, 0, 1, -1)) * C8);
-    acc += tp(5, 0, 0, 0) * (-(tp(2, 0, 0, 1) - tp(2, 0, 0, -1)) * C2 - 2 * Dsum);
-    // Us_w(P) = u(P+x) + u(P) + u(P+x-z) + u(P-z), at P = Q -+ x
-    const double usm = tp(0, 0, 0, 0) + tp(0, -1, 0, 0) + tp(0, 0, 0, -1) + tp(0, -1, 0, -1);
-    const double usp = tp(0, 2, 0, 0) + tp(0, 1, 0, 0) + tp(0, 2, 0, -1) + tp(0, 1, 0, -1);
-    acc += tp(5, -1, 0, 0) * (-usm * A8 + Dx);
-    acc += tp(5, 1, 0, 0) * (usp * A8 + Dx);
-    // Vs_w(P) = v(P+y) + v(P) + v(P+y-z) + v(P-z), at P = Q -+ y
-    const double vsm = tp(1, 0, 0, 0) + tp(1, 0, -1, 0) + tp(1, 0, 0, -1) + tp(1, 0, -1, -1);
-    const double vsp = tp(1, 0, 2, 0) + tp(1, 0, 1, 0) + tp(1, 0, 2, -1) + tp(1, 0, 1, -1);
-    acc += tp(5, 0, -1, 0) * (-vsm * B8 + Dy);
-    acc += tp(5, 0, 1, 0) * (vsp * B8 + Dy);
-    acc += tp(5, 0, 0, -1) * (-tp(2, 0, 0, -1) * C2 + Dz);
-    acc += tp(5, 0, 0, 1) * (tp(2, 0, 0, 1) * C2 + Dz);
-    XB2[o] = (T)acc;
-  }
-  // p_bar += b G^T z_bar at pressure points
-  if (i < g.N[0] && j < g.N[1] && k < g.N[2]) {
-    double acc = 0;
-    acc += (zt(0, 1, 0, 0) - zt(0, 0, 0, 0)) * g.one_over_h[0];
-    acc += (zt(1, 0, 1, 0) - zt(1, 0, 0, 0)) * g.one_over_h[1];
-    acc += (zt(2, 0, 0, 1) - zt(2, 0, 0, 0)) * g.one_over_h[2];
-    P[o] = (T)((double)P[o] + bcoef * acc);
-  }
-}
-
-// A 64 x 4 workgroup owns an (i, j) tile of the union of the component
-// extents and marches KB planes along k.  Planes k-1, k, k+1 of X and N_bar
-// (one-point halo in i and j) live in an LDS ring; plane k+2 is fetched
-// into registers while plane k is computed.  The few reach-2 taps of X and
-// the z_bar, p_bar accesses go to global memory.  Ring cells outside the
-// array hold zero: wherever N_bar is non-zero (component interiors) every X
-// tap of its term is an array point, so those zeros only meet N_bar = 0.
-// (256^3 FP64, 8 adjoint steps: 64 x 4 tiles of 4 planes 54.9 ms, 8 planes
-// 53.9, 16 planes 53.7; 64 x 8 tiles 55.8 (4 planes) and 55.1 (8 planes):
-// the kernel is not bound by its halo loads.  Every tap read from global
-// memory instead of the ring measured slower.)
-constexpr int AXT = 64, AYT = 4, AKB = 4;
-constexpr int AHX = AXT + 2, AHY = AYT + 2;
-constexpr int APL = AHY * AHX;                         // one field of a ring plane
-constexpr int ARH = (APL + AXT * AYT - 1) / (AXT * AYT);  // elements per thread and field
-
-template <typename T>
-__global__ void __launch_bounds__(AXT * AYT) k_adj_xb(DGrid g, Layout L, AdjVec Xv, AdjVec Nbv, AdjVec Zv, AdjVec Xbv,
-                                                T* __restrict__ P, double bcoef, int ntx, int nty, int ntiles) {
-  __shared__ T ring[3][6][AHY][AHX];
-  const int tx = threadIdx.x % AXT, ty = threadIdx.x / AXT, tid = threadIdx.x;
-  const int tile = xcd_tile(blockIdx.x, ntiles);
-  const int bx = tile % ntx, by = (tile / ntx) % nty, bz = tile / (ntx * nty);
-  const int i0 = bx * AXT, j0 = by * AYT, k0 = bz * AKB;
-  const int kend = min(k0 + AKB, g.N[2] + 1);
-  const int i = i0 + tx, j = j0 + ty;
-  const T* F[6] = {(const T*)Xv.f[0], (const T*)Xv.f[1], (const T*)Xv.f[2],
-                   (const T*)Nbv.f[0], (const T*)Nbv.f[1], (const T*)Nbv.f[2]};
-  // this thread's elements of every field of a ring plane: the same (ii, jj)
-  // positions in each of the six fields, so the field pointer is uniform
-  int off[ARH], lds[ARH];
-  bool ok[ARH];
-#pragma unroll
-  for (int h = 0; h < ARH; h++) {
-    const int q = tid + AXT * AYT * h;
-    const int jj = q / AHX, ii = q - jj * AHX;
-    const int gi = i0 - 1 + ii, gj = j0 - 1 + jj;
-    ok[h] = q < APL && gi >= 0 && gj >= 0 && gi < L.PX && gj < L.SY;
-    off[h] = ok[h] ? (int)L.idx(gi, gj, 0) : 0;
-    lds[h] = q < APL ? q : -1;
-  }
-  // planes outside the array are fetched at plane 0 and zeroed, like the
-  // cells outside it, when committed (so no instruction waits for the loads
-  // before the commit)
-  auto fetch = [&](int k, T (&v)[6][ARH]) {
-    const long kk = k >= 0 && k < L.SZ ? (long)k * L.plane : 0;
-#pragma unroll
-    for (int f = 0; f < 6; f++)
-#pragma unroll
-      for (int h = 0; h < ARH; h++) v[f][h] = F[f][kk + off[h]];
-  };
-  auto slot_of = [](int k) { return (k + 3) % 3; };
-  auto commit = [&](int k, const T (&v)[6][ARH]) {
-    const int sl = slot_of(k);
-    const bool kin = k >= 0 && k < L.SZ;
-#pragma unroll
-    for (int f = 0; f < 6; f++)
-#pragma unroll
-      for (int h = 0; h < ARH; h++)
-        if (lds[h] >= 0) (&ring[sl][f][0][0])[lds[h]] = ok[h] && kin ? v[f][h] : (T)0;
-  };
-  {
-    T a[6][ARH];
-    fetch(k0 - 1, a);
-    commit(k0 - 1, a);
-    fetch(k0, a);
-    commit(k0, a);
-    fetch(k0 + 1, a);
-    commit(k0 + 1, a);
-  }
-  T pre[6][ARH];
-  if (k0 + 2 <= kend) fetch(k0 + 2, pre);
+  // X, f at this thread's point of plane k, displaced within the plane
+  auto xat = [&](int k, int c, int di, int dj) -> double { return (double)xs[k & 1][c][ty + 1 + dj][tx + 1 + di]; };
+  // planes k0-2 (what plane k0-1 needs of it), then k0-1 and k0 into LDS
+  double su0, sv0, x0[3];  // of the plane below: u(P) + u(P+x), v(P) + v(P+y), X(P)
+  fetch_x(k0 - 2);
+  commit_x(k0 - 2);
+  fetch_x(k0 - 1);
+  commit_x(k0 - 1);
+  fetch_x(k0);
+  fetch_n(k0 - 1);
   __syncthreads();
+#pragma unroll
+  for (int c = 0; c < 3; c++) x0[c] = xat(k0, c, 0, 0);  // (the slot of plane k0-2)
+  su0 = x0[0] + xat(k0, 0, 1, 0);
+  sv0 = x0[1] + xat(k0, 1, 0, 1);
+  __syncthreads();
+  commit_x(k0);
 
-  const bool in_tile = i <= g.N[0] && j <= g.N[1];
-  const long last = L.elems - 1;
-  const long PX = L.PX, PL = L.plane;
-  for (int k = k0; k < kend; k++) {
-    if (in_tile) {
-      const long o = L.idx(i, j, k);
-      const int sl[3] = {slot_of(k - 1), slot_of(k), slot_of(k + 1)};
-      auto tp = [&](int f, int di, int dj, int dk) -> double {
-        if (di >= -1 && di <= 1 && dj >= -1 && dj <= 1 && dk >= -1 && dk <= 1)
-          return (double)ring[sl[dk + 1]][f][ty + 1 + dj][tx + 1 + di];
-        long idx = o + di + PX * dj + PL * dk;
-        idx = idx < 0 ? 0 : (idx > last ? last : idx);
-        return (double)F[f][idx];
-      };
-      auto zt = [&](int c, int di, int dj, int dk) -> double {
-        long idx = o + di + PX * dj + PL * dk;
-        idx = idx < 0 ? 0 : (idx > last ? last : idx);
-        return (double)((const T*)Zv.f[c])[idx];
-      };
-      adj_xb_point<T>(g, o, i, j, k, tp, zt, (T*)Xbv.f[0], (T*)Xbv.f[1], (T*)Xbv.f[2], P, bcoef);
+  // acc: the outputs of plane m-1 but for what plane m adds; dn: what plane
+  // m-1 adds to plane m
+  double acc[3] = {0, 0, 0}, dn[3] = {0, 0, 0};
+  for (int m = k0 - 1; m <= kend; m++) {
+    __syncthreads();
+    double n[3];
+#pragma unroll
+    for (int c = 0; c < 3; c++) n[c] = own && plane_ok(m) ? (double)pn[c] : 0.0;
+    // memory requests in the order their values are waited for: the operands
+    // of output plane m-1, then plane m+2 of X and m+1 of N_bar, which stay in
+    // flight until the next plane
+    const int k = m - 1;
+    const bool emit = out && k >= k0;
+    const long kp = plane_at(k);
+    double z[3], zn[3], pv;
+#pragma unroll
+    for (int c = 0; c < 3; c++) z[c] = (double)(Z[c] + kp)[lane(oo)];
+    const unsigned az = lane(oz);
+    zn[1] = (double)(Z[1] + kp)[az + L.PX];
+    zn[2] = (double)(Z[2] + plane_at(k + 1))[az];
+    pv = (double)(P + kp)[az];
+    fetch_x(m + 2);
+    fetch_n(m + 1);
+    // products of plane m
+    const double u = xat(m, 0, 0, 0), v = xat(m, 1, 0, 0), w = xat(m, 2, 0, 0);
+    double here[3] = {dn[0] - D2 * n[0], dn[1] - D2 * n[1], dn[2] - D2 * n[2]};
+    double fv_x, fw_x, fw_y, fu_y, su, sv, swx, swy;
+    {
+      const double up = xat(m, 0, 1, 0), ud = xat(m, 0, 0, -1);
+      su = u + up;
+      here[0] -= A2 * n[0] * (up - xat(m, 0, -1, 0));
+      fu_y = n[0] * (xat(m, 0, 0, 1) - ud);
+      pr[PH_VU][ty][tx] = n[1] * (su + xat(m, 0, 1, -1) + ud);
     }
+    {
+      const double vp = xat(m, 1, 0, 1), vl = xat(m, 1, -1, 0);
+      sv = v + vp;
+      here[1] -= B2 * n[1] * (vp - xat(m, 1, 0, -1));
+      fv_x = n[1] * (xat(m, 1, 1, 0) - vl);
+      pr[PH_UV][ty][tx] = n[0] * (sv + xat(m, 1, -1, 1) + vl);
+    }
+    {
+      const double wl = xat(m, 2, -1, 0), wd = xat(m, 2, 0, -1);
+      swx = w + wl;
+      swy = w + wd;
+      fw_x = n[2] * (xat(m, 2, 1, 0) - wl);
+      fw_y = n[2] * (xat(m, 2, 0, 1) - wd);
+    }
+    const double gu = n[0] * u, gw = n[2] * w;
+#pragma unroll
+    for (int c = 0; c < 3; c++) pr[PN_U + c][ty][tx] = n[c];
+    pr[PG_V][ty][tx] = n[1] * v;
+    pr[PH_WU][ty][tx] = n[2] * (su + su0);
+    pr[PH_WV][ty][tx] = n[2] * (sv + sv0);
+    pr[PF_UY][ty][tx] = fu_y;
+    pr[PF_VX][ty][tx] = fv_x;
+    pr[PF_WY][ty][tx] = fw_y;
+    double fu_z, fv_z, hu_w, hv_w;
+    {
+      const double u1 = xat(m + 1, 0, 0, 0), v1 = xat(m + 1, 1, 0, 0), w1 = xat(m + 1, 2, 0, 0);
+      hu_w = n[0] * (swx + w1 + xat(m + 1, 2, -1, 0));
+      hv_w = n[1] * (swy + w1 + xat(m + 1, 2, 0, -1));
+      fu_z = n[0] * (u1 - x0[0]);
+      fv_z = n[1] * (v1 - x0[1]);
+      here[2] -= C2 * n[2] * (w1 - x0[2]);
+    }
+    pr[PF_VZ][ty][tx] = fv_z;
+    x0[0] = u;
+    x0[1] = v;
+    x0[2] = w;
+    su0 = su;
+    sv0 = sv;
+    // x neighbours lie in the same wave (a wave is two rows of 32 points)
+    const double fw_xl = __shfl_up(fw_x, 1, 64), fu_zr = __shfl_down(fu_z, 1, 64);
+    zn[0] = __shfl_down(z[0], 1, 64);
+    const double gu_l = __shfl_up(gu, 1, 64), gu_r = __shfl_down(gu, 1, 64);
     __syncthreads();
-    // plane k+2 replaces plane k-1; plane k+3 starts loading
-    if (k + 2 <= kend) commit(k + 2, pre);
-    if (k + 3 <= kend) fetch(k + 3, pre);
-    __syncthreads();
+    if (out) {
+      auto at = [&](int f, int di, int dj) -> double { return pr[f][ty + dj][tx + di]; };
+      const double t1 = fw_x + fw_xl, t2 = fw_y + at(PF_WY, 0, -1);
+      const double t3 = fu_z + fu_zr + fv_z + at(PF_VZ, 0, 1);
+      // outputs of plane m-1
+      if (emit) {
+        const double ub = acc[0] + (C8 * hu_w + Dz * n[0] - A8 * t1) + z[0];
+        const double vb = acc[1] + (C8 * hv_w + Dz * n[1] - B8 * t2) + z[1];
+        const double wb = acc[2] + (C2 * gw + Dz * n[2]) + z[2];
+        if (in_field(g, 0, i, j, k)) ((T*)Xbv.f[0] + kp)[lane(oo)] = (T)ub;
+        if (in_field(g, 1, i, j, k)) ((T*)Xbv.f[1] + kp)[lane(oo)] = (T)vb;
+        if (in_field(g, 2, i, j, k)) ((T*)Xbv.f[2] + kp)[lane(oo)] = (T)wb;
+        if (pcol && k < g.N[2])
+          (P + kp)[lane(oz)] = (T)(pv + bcoef * ((zn[0] - z[0]) * g.one_over_h[0] + (zn[1] - z[1]) * g.one_over_h[1] +
+                                   (zn[2] - z[2]) * g.one_over_h[2]));
+      }
+      // plane m from its own products
+      auto lap = [&](int f) { return Dx * (at(f, 1, 0) + at(f, -1, 0)) + Dy * (at(f, 0, 1) + at(f, 0, -1)); };
+      acc[0] = here[0] + lap(PN_U) + A2 * (gu_r - gu_l) +
+               B8 * (at(PH_UV, 0, 1) - at(PH_UV, 0, -1)) -
+               A8 * ((fv_x + at(PF_VX, -1, 0) + at(PF_VX, 0, 1) + at(PF_VX, -1, 1)) + t1);
+      acc[1] = here[1] + lap(PN_V) + B2 * (at(PG_V, 0, 1) - at(PG_V, 0, -1)) +
+               A8 * (at(PH_VU, 1, 0) - at(PH_VU, -1, 0)) -
+               B8 * ((fu_y + at(PF_UY, 0, -1) + at(PF_UY, 1, 0) + at(PF_UY, 1, -1)) + t2);
+      acc[2] = here[2] + lap(PN_W) + A8 * (at(PH_WU, 1, 0) - at(PH_WU, -1, 0)) +
+               B8 * (at(PH_WV, 0, 1) - at(PH_WV, 0, -1)) - C8 * t3;
+      dn[0] = Dz * n[0] - C8 * hu_w;
+      dn[1] = Dz * n[1] - C8 * hv_w;
+      dn[2] = Dz * n[2] - C2 * gw - C8 * t3;
+    }
+    // plane m+2 takes the slot of plane m, which every thread has read
+    commit_x(m + 2);
   }
 }
 
@@ -452,17 +511,37 @@ __global__ void __launch_bounds__(AXT * AYT) k_adj_xb(DGrid g, Layout L, AdjVec 
 template <typename T>
 void launch_adj_rhs(const DGrid& g, const Layout& L, const T* P, const AdjVec& Y, double dts, T* B, long bp0,
                     long bplane, hipStream_t st) {
-  const long total = (long)g.npts[0] * g.npts[1] * g.npts[2];
-  k_adj_rhs<T><<<(unsigned)((total + 255) / 256), 256, 0, st>>>(g, L, P, Y, dts, B, bp0, bplane, total);
+  const int nx = (g.npts[0] + 63) / 64, items = nx * g.npts[1] * g.npts[2];
+  k_adj_rhs<T><<<(unsigned)((items + 3) / 4), 256, 0, st>>>(g, L, P, Y, dts, B, bp0, bplane, nx, items);
 }
+
+// Rows per plane, 64-point items per row and items of k_adj_zb: the union of
+// the components' interiors.
+struct ZbShape {
+  int rows, nx, items;
+};
+static ZbShape zb_shape(const DGrid& g) {
+  int top[3] = {0, 0, 0};
+  for (int c = 0; c < 3; c++) {
+    int e[3];
+    extents(g, c, e);
+    for (int ax = 0; ax < 3; ax++) top[ax] = std::max(top[ax], e[ax] - 2);
+  }
+  const int nx = (top[0] + 63) / 64;
+  return {top[1], nx, nx * top[1] * top[2]};
+}
+
+int adj_zb_blocks(const DGrid& g) { return std::clamp((zb_shape(g).items + 3) / 4, 1, kAdjMaxBlocks); }
 
 template <typename T>
 void launch_adj_zb(const DGrid& g, const Layout& L, const AdjVec& Y, const T* Bpsi, long bp0, long bplane, double dts,
                    const AdjVec& Zb, const AdjVec& Nb, const AdjVec& Zo, double alpha, double beta, double fcoef,
                    int accumulate, double* partial,
                    int nblk, hipStream_t st) {
-  k_adj_zb<T><<<dim3(nblk, 3, 1), 256, 0, st>>>(g, L, Y, Bpsi, bp0, bplane, dts, Zb, Nb, Zo, alpha, beta, fcoef,
-                                                accumulate, partial);
+  const ZbShape sh = zb_shape(g);
+  k_adj_zb<T><<<nblk, 256, 0, st>>>(g, L, Y, Bpsi, bp0, bplane, g.one_over_h[0] / dts, g.one_over_h[1] / dts,
+                                    g.one_over_h[2] / dts, Zb, Nb, Zo, alpha, beta, fcoef, accumulate, partial,
+                                    sh.rows, sh.nx, sh.items);
 }
 
 void launch_adj_sum(const double* partial, int nblk, int accumulate, double* out, hipStream_t st) {
@@ -473,10 +552,15 @@ template <typename T>
 void launch_adj_xb(const DGrid& g, const Layout& L, const AdjVec& X, const AdjVec& Nb, const AdjVec& Zb,
                    const AdjVec& Xb, T* P, double bcoef, hipStream_t st) {
   // tiles over points 0..N per axis
-  const int ntx = (g.N[0] + 1 + AXT - 1) / AXT, nty = (g.N[1] + 1 + AYT - 1) / AYT;
-  const int ntz = (g.N[2] + 1 + AKB - 1) / AKB;
-  const int ntiles = ntx * nty * ntz;
-  k_adj_xb<T><<<ntiles, AXT * AYT, 0, st>>>(g, L, X, Nb, Zb, Xb, P, bcoef, ntx, nty, ntiles);
+  const int ntx = (g.N[0] + AOX) / AOX, nty = (g.N[1] + AOY) / AOY;
+  // planes per workgroup: each chunk repeats two planes of products, and a
+  // chunk's planes are a serial chain of about 2.6 us each.  Adjoint step, 2 / 4
+  // / 6 / 16 planes: 32^3 317 / 333 / 353 / 433 us, 64^3 419 / 410 / 423 / 498, 96^3
+  // 637 / 603 / 592 / 622, 128^3 1115 / 1036 / 1023 / 1009, 256^3 6.27 / 5.60 /
+  // 5.41 / 5.15 ms
+  const int kchunk = (int)std::clamp((long)ntx * nty * (g.N[2] + 1) / 400, 2L, 16L);
+  const int ntiles = ntx * nty * ((g.N[2] + kchunk) / kchunk);
+  k_adj_xb<T><<<ntiles, AXT * AYT, 0, st>>>(g, L, X, Nb, Zb, Xb, P, bcoef, ntx, nty, ntiles, kchunk);
 }
 
 #define MIF_ADJ_INST(T)                                                                                              \

@@ -936,8 +936,7 @@ int step_adjoint(mif_ctx* c, mif_field* const un[3], mif_field* const y2[3], mif
   const AdjVec zlater[4] = {AdjVec{}, ZB, ZA, ZA};
   T* P = fptr<T>(pbar);
   T* B = (T*)c->B;
-  const long interior_pts = (long)(g.N[0] + 1) * (g.N[1] + 1) * (g.N[2] + 1);
-  const int nblk = (int)std::min<long>(kAdjMaxBlocks, (interior_pts + 255) / 256);
+  const int nblk = adj_zb_blocks(g);
   KTimer tm(c, MIF_KC_ADJOINT);
   for (int s = 3; s >= 1; s--) {
     const AdjVec Yin = s == 3 ? UB : XT;

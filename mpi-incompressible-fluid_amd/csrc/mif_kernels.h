@@ -253,9 +253,10 @@ template <typename T>
 void launch_adj_zb(const DGrid& g, const Layout& L, const AdjVec& Y, const T* Bpsi, long bp0, long bplane, double dts,
                    const AdjVec& Zb, const AdjVec& Nb, const AdjVec& Zo, double alpha, double beta, double fcoef,
                    int accumulate, double* partial, int nblk, hipStream_t st);
-// Workgroups per component of k_adj_zb (one point per thread up to this
-// many, grid-stride beyond), and the number of partials k_adj_sum reduces.
+// Workgroups of k_adj_zb (64 points per wave up to this many, grid-stride
+// beyond), and the number of partials per component k_adj_sum reduces.
 constexpr int kAdjMaxBlocks = 4096;
+int adj_zb_blocks(const DGrid& g);
 // out[c] = (accumulate: out[c] +) the sum of the nblk <= kAdjMaxBlocks
 // partials of component c.
 void launch_adj_sum(const double* partial, int nblk, int accumulate, double* out, hipStream_t st);
