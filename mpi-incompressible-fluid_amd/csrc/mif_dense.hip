@@ -79,7 +79,7 @@ struct Mm<float> {
 constexpr int NL = 16;
 
 // What the x pass loads or stores instead of its buffer (FusedIO).
-enum { IO_PLAIN = 0, IO_FIELD = 1, IO_FIELD_DC = 2, IO_DEFECT = 3 };
+enum { IO_PLAIN = 0, IO_FIELD = 1, IO_FIELD_DC = 2, IO_DEFECT = 3, IO_PACK = 4 };
 
 }  // namespace dense
 
@@ -135,7 +135,7 @@ __global__ void __launch_bounds__(1024) k_dense(DGrid g, DensePlan P, const T* _
       const bool ok = r < n1 * n2;
       const int rj = ok ? r % n1 : 0, rk = ok ? r / n1 : 0;
       lbase[t] = ok ? bp0 * rj + bplane * rk : -1;
-      if constexpr (IO == IO_FIELD || IO == IO_FIELD_DC) {
+      if constexpr (IO == IO_FIELD || IO == IO_FIELD_DC || IO == IO_PACK) {
         const int j = rj + g.olo[1], k = rk + g.olo[2];
         if constexpr (MODE == 0) {
           lrow[t][0] = ok ? io.L.idx(g.olo[0], j, k) : -1;
@@ -168,6 +168,8 @@ __global__ void __launch_bounds__(1024) k_dense(DGrid g, DensePlan P, const T* _
       const long b = lbase[l];
       if constexpr (IO == IO_PLAIN) {
         return B[(b >= 0 ? b : 0) + m];
+      } else if constexpr (IO == IO_PACK) {
+        return ((const T*)io.P)[(b >= 0 ? lrow[l][0] : 0) + m];
       } else if constexpr (IO == IO_DEFECT) {
         // r = (b - mean) - L phi in FP64 with the 7-point operator
         const float* F = io.phi32;
@@ -537,6 +539,8 @@ void launch_dense(const DGrid& g, int axis, int mode, const DensePlan& P, const 
   } else if (!io) {
     if (mode == 0) launch_dense_pass<T, 0, 0, IO_PLAIN, T>(g, P, sc, B, bp0, bplane, none, st);
     else launch_dense_pass<T, 0, 1, IO_PLAIN, T>(g, P, sc, B, bp0, bplane, none, st);
+  } else if (io->pack && mode == 0) {
+    launch_dense_pass<T, 0, 0, IO_PACK, T>(g, P, sc, B, bp0, bplane, *io, st);
   } else if (sizeof(T) == 4 && io->res) {
     if constexpr (sizeof(T) == 4) launch_dense_pass<T, 0, 0, IO_DEFECT, T>(g, P, sc, B, bp0, bplane, *io, st);
   } else if (sizeof(T) == 4 && io->dc) {

@@ -303,6 +303,18 @@ __global__ void __launch_bounds__(256) k_fft_p2(DGrid g, const T* __restrict__ W
     yzrow[t][2] = bp0 * j + bplane * nb(g, 2, k, -1);
     yzrow[t][3] = bp0 * j + bplane * nb(g, 2, k, 1);
   }
+  // plain x forward pass: the rows it reads, of its buffer or of the field the
+  // right-hand side sits in (FusedIO::pack)
+  constexpr bool SRC = AXIS == 0 && MODE == 0 && !FUSED && !RES;
+  __shared__ long srow[SRC ? 2 * NP : 1];
+  const T* src = SRC && io.pack ? (const T*)io.P : B;
+  if (SRC && t < NL) {
+    const int r = bx * NL + t;
+    if (r >= n1 * n2)
+      srow[t] = -1;
+    else
+      srow[t] = io.pack ? io.L.idx(g.olo[0], r % n1 + g.olo[1], r / n1 + g.olo[2]) : bp0 * (r % n1) + bplane * (r / n1);
+  }
   if (t < NL) {
     long b = -1;
     if (AXIS == 0) {
@@ -399,7 +411,7 @@ __global__ void __launch_bounds__(256) k_fft_p2(DGrid g, const T* __restrict__ W
 #pragma unroll
       for (int a = 0; a < CL; a++) {
         const int l = l0 + a;
-        const long b = l < NL ? lbase[l] : -1;
+        const long b = l < NL ? (SRC ? srow[l] : lbase[l]) : -1;
         if constexpr (RES) {
           // r = (b - mean) - (lx + ly + lz) in FP64, the 7-point operator
           // scaled by 1/h^2; a line outside the grid reads row 0 and is dropped
@@ -425,7 +437,7 @@ __global__ void __launch_bounds__(256) k_fft_p2(DGrid g, const T* __restrict__ W
         for (int q = 0; q < R0; q++) {
           const int m = t + 256 * q;
           const bool okm = b >= 0 && m < n;
-          const T x = B[okm ? b + m : 0];
+          const T x = src[okm ? b + m : 0];
           val[a][q] = okm ? x : (T)0;
         }
       }
@@ -1053,7 +1065,9 @@ static void launch_p2(const DGrid& g, int axis, int mode, const FftPlan& plan, c
   const int per = plan.periodic;
 #define MIF_P2(AX, MD) k_fft_p2<T, L, NP, AX, MD, false><<<grd, 256, 0, st>>>(g, W, sc, B, bp0, bplane, per, none)
   if constexpr (PASSES & 1) {
-    if (axis == 0 && io && io->res) {
+    if (axis == 0 && io && io->pack && mode == 0) {
+      k_fft_p2<T, L, NP, 0, 0, false><<<grd, 256, 0, st>>>(g, W, sc, B, bp0, bplane, per, *io);
+    } else if (axis == 0 && io && io->res) {
       if constexpr (sizeof(T) == 4)
         k_fft_p2<T, L, NP, 0, 0, false, T, false, true><<<grd, 256, 0, st>>>(g, W, sc, B, bp0, bplane, per, *io);
     } else if (axis == 0 && io && io->dc) {

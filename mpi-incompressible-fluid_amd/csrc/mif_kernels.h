@@ -111,6 +111,9 @@ struct FusedIO {
   // the velocity and pressure fields hold FP32 values while the transform
   // runs in FP64 (the mixed form with FP64 transforms)
   int fields_fp32 = 0;
+  // x forward pass of a right-hand side held in the pressure field P: it reads
+  // the field's owner points (element type T) in place of its buffer
+  int pack = 0;
   // mixed form with one FP64 defect sweep (FP32 transforms): the forward
   // pass also stores the FP64 divergence b (packed layout) and per-workgroup
   // owner-weighted sums (W.b, W.1) into partial; the inverse pass adds the
