@@ -460,8 +460,8 @@ k_stage(DGrid g, Layout L, StageArgs s, VelStageArgs vs, int imax, int jmax, int
 #pragma unroll
         for (int c = 0; c < 3; c++)
           if (inside[c]) {
-            av[c] = ((const T*)vs.R[c])[ol];
-            if constexpr (KIND == 5) bv[c] = ((const T*)vs.V[c])[ol];
+            av[c] = load_in<NT && kNtLoads>(&((const T*)vs.R[c])[ol]);
+            if constexpr (KIND == 5) bv[c] = load_in<NT && kNtLoads>(&((const T*)vs.V[c])[ol]);
           }
       }
     };
@@ -555,13 +555,13 @@ k_stage(DGrid g, Layout L, StageArgs s, VelStageArgs vs, int imax, int jmax, int
           }
           const T f = rhs + (T)fc;
           if constexpr (KIND == 4) {
-            ((T*)vs.R[c])[o] = f;
-            ((T*)vs.B[c])[o] = x + dt * (T)(8.0 / 15.0) * f;
+            store_out<NT>(&((T*)vs.R[c])[o], f);
+            store_out<NT>(&((T*)vs.B[c])[o], x + dt * (T)(8.0 / 15.0) * f);
           } else if constexpr (KIND == 5) {
-            ((T*)vs.R[c])[o] = bv[c] + dt * ((T)(1.0 / 4.0) * av[c]);
-            ((T*)vs.V[c])[o] = bv[c] + dt * ((T)(1.0 / 4.0) * av[c] + (T)(5.0 / 12.0) * f);
+            store_out<NT>(&((T*)vs.R[c])[o], bv[c] + dt * ((T)(1.0 / 4.0) * av[c]));
+            store_out<NT>(&((T*)vs.V[c])[o], bv[c] + dt * ((T)(1.0 / 4.0) * av[c] + (T)(5.0 / 12.0) * f));
           } else {
-            ((T*)vs.B[c])[o] = av[c] + dt * ((T)(3.0 / 4.0) * f);
+            store_out<NT>(&((T*)vs.B[c])[o], av[c] + dt * ((T)(3.0 / 4.0) * f));
           }
         }
       }
@@ -1301,16 +1301,35 @@ void launch_stage(int stage, const DGrid& g, const Layout& L, const StageArgs& s
     L.nt ? launch_stage_kind<T, 3, false, true>(g, L, s, vs, st) : launch_stage_kind<T, 3>(g, L, s, vs, st);
 }
 
+// The velocity-only kinds read 6 to 9 arrays and write 3 to 6, and are bound by
+// that traffic once the fields are larger than the cache.  Streamed past it
+// (stage kernel, mean of a step's three, ordinary -> non-temporal): 256^3
+// nodes FP64 409 -> 383 us, 300^3 689 -> 651, 190^3 179 -> 168, 172^3 (43 MB
+// fields) 148 -> 138, 160^3 (36 MB) 118.4 -> 118.5; mixed 256^3 250 -> 245,
+// 224^3 202 -> 197, 208^3 (41 MB) 162.6 -> 159.3, 200^3 (37 MB) 153.6 ->
+// 155.2, 192^3 (33 MB) 137 -> 142.  The line lies between the last two
+// groups, a little above the full step's, which streams more arrays.
+constexpr long kVelNtMinFieldBytes = 40L << 20;
+
 template <typename T>
 void launch_vel_stage(int stage, const DGrid& g, const Layout& L, const VelStageArgs& vs, hipStream_t st) {
   StageArgs s{};
-  const bool ft = vs.forcing.kind == MIF_FN_VT_FORCING;
-  if (stage == 1)
-    ft ? launch_stage_kind<T, 4, true>(g, L, s, vs, st) : launch_stage_kind<T, 4>(g, L, s, vs, st);
-  else if (stage == 2)
-    ft ? launch_stage_kind<T, 5, true>(g, L, s, vs, st) : launch_stage_kind<T, 5>(g, L, s, vs, st);
+  auto go = [&](auto ft, auto nt) {
+    constexpr bool F = decltype(ft)::value, N = decltype(nt)::value;
+    if (stage == 1)
+      launch_stage_kind<T, 4, F, N>(g, L, s, vs, st);
+    else if (stage == 2)
+      launch_stage_kind<T, 5, F, N>(g, L, s, vs, st);
+    else
+      launch_stage_kind<T, 6, F, N>(g, L, s, vs, st);
+  };
+  using yes = std::true_type;
+  using no = std::false_type;
+  const bool nt = L.nt && L.elems * (long)sizeof(T) > kVelNtMinFieldBytes;
+  if (vs.forcing.kind == MIF_FN_VT_FORCING)
+    nt ? go(yes{}, yes{}) : go(yes{}, no{});
   else
-    ft ? launch_stage_kind<T, 6, true>(g, L, s, vs, st) : launch_stage_kind<T, 6>(g, L, s, vs, st);
+    nt ? go(no{}, yes{}) : go(no{}, no{});
 }
 
 __global__ void __launch_bounds__(256) k_axis_tables(DGrid g, double* __restrict__ tab, int n) {
