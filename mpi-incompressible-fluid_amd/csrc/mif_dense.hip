@@ -30,10 +30,12 @@
 // through the other three workgroups of its CU.
 //
 // Work split: a workgroup owns 16 lines; each wave owns one of the
-// H / 16 row tiles (H = R/2 + 1) of both matrices, for all lines.  The
+// H / 16 row tiles (H = R/2 + 1) of both matrices, for all lines (on x there
+// may be waves beyond those, launch_dense_pass).  The
 // folded lines (e and o) sit in LDS, the matrices are read fragment by
 // fragment from global memory (they are shared by all workgroups and stay in
 // L2; a fragment is one 16-byte load per lane in FP64).
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -123,8 +125,9 @@ __global__ void __launch_bounds__(1024) k_dense(DGrid g, DensePlan P, const T* _
   };
 
   // ---- load, folded
-  // x pass: lines are rows (j, k); a group of 2^lg lanes reads one line
-  const int lg = H <= 16 ? 4 : (H <= 32 ? 5 : 6);
+  // x pass: lines are rows (j, k), their points dealt to the threads in order;
+  // q / KP by its reciprocal, exact for q < 16 KP <= 4096
+  const unsigned rkp = (1u << 22) / KP + 1;
   __shared__ long lrow[AXIS == 0 ? NL : 1][4];
   __shared__ long lbase[AXIS == 0 ? NL : 1];
   __shared__ double lwt[IO == IO_FIELD_DC ? NL : 1];
@@ -199,35 +202,31 @@ __global__ void __launch_bounds__(1024) k_dense(DGrid g, DensePlan P, const T* _
         return (T)bv;
       }
     };
-    const int j0 = t & ((1 << lg) - 1);
-    for (int l = t >> lg; l < NL; l += nthr >> lg) {
+    for (int q = t; q < NL * KP; q += nthr) {
+      const int l = (q * rkp) >> 22, j = q - l * KP;
       const bool ok = lbase[l] >= 0;
-      for (int j = j0; j < KP; j += 1 << lg) {
-        T e = 0, o = 0;
-        if (j < H) {
-          const T a = value(l, j);
-          if (self(j)) {
-            e = ok ? a : (T)0;
-          } else {
-            const T b = value(l, R - j);
-            e = ok ? a + b : (T)0;
-            o = ok ? a - b : (T)0;
-          }
+      T e = 0, o = 0;
+      if (j < H) {
+        const T a = value(l, j);
+        if (self(j)) {
+          e = ok ? a : (T)0;
+        } else {
+          const T b = value(l, R - j);
+          e = ok ? a + b : (T)0;
+          o = ok ? a - b : (T)0;
         }
-        Eo[at(j, l)] = e;
-        Eo[half + at(j, l)] = o;
       }
+      Eo[at(j, l)] = e;
+      Eo[half + at(j, l)] = o;
     }
   } else if constexpr (AXIS == 0) {
-    const int r0 = t & ((1 << lg) - 1);
-    for (int l = t >> lg; l < NL; l += nthr >> lg) {
+    for (int q = t; q < NL * KP; q += nthr) {
+      const int l = (q * rkp) >> 22, r = q - l * KP;
       const long b = lbase[l];
-      for (int r = r0; r < KP; r += 1 << lg) {
-        const int se = slot_e(r), so = slot_o(r);
-        const T e = B[b >= 0 && se >= 0 ? b + se : 0], o = B[b >= 0 && so >= 0 ? b + so : 0];
-        Eo[at(r, l)] = b >= 0 && se >= 0 ? e : (T)0;
-        Eo[half + at(r, l)] = b >= 0 && so >= 0 ? o : (T)0;
-      }
+      const int se = slot_e(r), so = slot_o(r);
+      const T e = B[b >= 0 && se >= 0 ? b + se : 0], o = B[b >= 0 && so >= 0 ? b + so : 0];
+      Eo[at(r, l)] = b >= 0 && se >= 0 ? e : (T)0;
+      Eo[half + at(r, l)] = b >= 0 && so >= 0 ? o : (T)0;
     }
   } else {
     const int l = t & (NL - 1), step = nthr / NL;
@@ -281,7 +280,8 @@ __global__ void __launch_bounds__(1024) k_dense(DGrid g, DensePlan P, const T* _
   // 120-283 nodes is then that of the mixed-radix transform (2e-7; 3e-7 with
   // the FP64 scheme)
   Acc acc[2][2];
-  const int MT = P.MT;
+#pragma unroll
+  for (int c = 0; c < 4; c++) acc[c >> 1][c & 1] = Acc{0, 0, 0, 0};
   auto multiply = [&](const T* Me) {
     const T* Mo = Me + (long)P.MT * KS * 128;
 #pragma unroll
@@ -322,7 +322,8 @@ __global__ void __launch_bounds__(1024) k_dense(DGrid g, DensePlan P, const T* _
     acc[1][0] += acc[1][1];
   };
   const long msize = 2L * P.MT * KS * 128;  // one direction's two matrices
-  multiply(M + (MODE == 1 ? msize : 0));
+  // the x passes may have waves without a row tile: they load and store only
+  if (AXIS != 0 || wave < P.MT) multiply(M + (MODE == 1 ? msize : 0));
 
   if constexpr (MODE == 2) {
     // scale every mode by 1/((lx+ly+lz) * norm), constant mode -> 0, and
@@ -386,6 +387,8 @@ __global__ void __launch_bounds__(1024) k_dense(DGrid g, DensePlan P, const T* _
       }
     }
     __syncthreads();
+    // a group of 2^lg lanes stores one line
+    const int lg = H <= 16 ? 4 : (H <= 32 ? 5 : 6);
     const int m0 = t & ((1 << lg) - 1);
     for (int l = t >> lg; l < NL; l += nthr >> lg) {
       const long b = lbase[l];
@@ -523,7 +526,23 @@ static void launch_dense_pass(const DGrid& g, const DensePlan& P, const Spectral
   auto* kernel = k_dense<T, AXIS, MODE, IO, TV>;
   if (lds > 64 * 1024)
     (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  kernel<<<grd, 64 * P.MT, lds, st>>>(g, P, M, sc, B, bp0, bplane, io);
+  // One wave per row tile; on x more, which load and store lines only.  There
+  // a thread's loads wait for one another, point after point, so the pass
+  // lasts as long as one thread has points.  A power of two keeps the waves
+  // even over the 16 lines of the store; few workgroups get a thread per point
+  // of their lines, as long as the device then holds them all at once (4096
+  // waves).  Divergence / unpack pass, one wave per row tile -> this rule and
+  // the points spread evenly over the threads (us): FP64 31^3 8.4 / 8.2 -> 6.3
+  // / 6.2, 65^3 11.9 / 11.9 -> 10.5 / 8.5, 96^3 15.8 / 13.2 -> 12.9 / 10.9,
+  // 151^3 42.7 / 31.2 -> 32.6 / 25.9, 181^3 61.6 / 45.0 -> 50.3 / 42.4, 301^3
+  // 351 / 256 -> 333 / 242; FP32 151^3 31.7 / 24.6 -> 24.6 / 20.5, 301^3 246 /
+  // 172 -> 210 / 159.
+  int waves = P.MT;
+  if (AXIS == 0) {
+    while (waves & (waves - 1)) waves++;
+    waves = std::max(waves, std::min({16, 2 * P.KS, 4096 / (int)grd.x}));
+  }
+  kernel<<<grd, 64 * waves, lds, st>>>(g, P, M, sc, B, bp0, bplane, io);
 }
 
 template <typename T>

@@ -413,16 +413,18 @@ void launch_fft_axis(const DGrid& g, int axis, int dir, int fused, const FftPlan
 // that kernel holds 16 to 32 lines per workgroup there, and neither its
 // workgroups nor its threads fill the device while there are few lines.
 // Divergence / unpack pass, specialised -> products (us): FP64 64 periodic
-// points on 65^2 lines 13.4 / 15.2 -> 10.6 / 10.2, 129^2 16.6 / 17.2 -> 16.1 /
-// 13.8, 257^2 31.7 / 26.7 -> 40.8 / 30.4 (so not there); 33 and 49 wall nodes
-// at every line count, 257^2: 29.4 / 27.6 -> 25.2 / 20.1 and 44.0 / 24.5 -> 28.3
-// / 21.1; FP32 96 points on 129^2 17.5 / 16.7 -> 14.0 / 12.8; FP64 128 points
-// on 129^2 19.9 / 14.8 -> 24.5 / 19.1 (so FP64 lines of more than 65 points keep
-// theirs).
+// points on 65^2 lines 13.2 / 15.4 -> 7.8 / 7.3, 129^2 16.5 / 17.3 -> 14.3 /
+// 11.4, 257^2 32.1 / 26.0 -> 34.5 / 27.7 (so not there); 33 and 49 wall nodes
+// at every line count, 257^2: 29.0 / 26.8 -> 22.9 / 18.0 and 44.4 / 24.5 -> 28.3
+// / 20.3; FP32 96 points on 129^2 16.8 / 16.9 -> 13.8 / 12.8, 257^2 27.7 / 25.0
+// -> 35.0 / 30.3.  FP64 lines of more than 65 points only up to 8192 lines: 96
+// points on 65^2 11.1 / 11.4 -> 8.8 / 8.8, 128 points on 65^2 11.2 / 11.6 ->
+// 10.6 / 10.2, on 97^2 16.4 / 14.0 -> 18.2 / 14.2.
 bool dense_x_short(const DGrid& g, const FftPlan& plan, bool fp64) {
   if (!plan.dense.M64 || plan.L > 128 || !fft_fast_len(plan.L)) return false;
   if (!plan.periodic && plan.L <= 96) return true;
-  return !(fp64 && plan.n > 65) && pow2_x_blocks(g, plan, fp64) < 1500;
+  if (fp64 && plan.n > 65 && (long)g.npts[1] * g.npts[2] > 8192) return false;
+  return pow2_x_blocks(g, plan, fp64) < 1500;
 }
 
 bool fused_x_pass(const FftPlan& plan) { return fft_fast_len(plan.L) || plan.dense.M64; }
