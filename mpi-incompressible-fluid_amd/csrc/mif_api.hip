@@ -635,14 +635,24 @@ int finish_standalone_solve(mif_ctx* c, mif_field* p) {
 int pressure_solve_any(mif_ctx* c, mif_field* p, mif_field* const vel[3], double dt, const FnDesc& gp, double tg,
                        int nhn);
 
+template <typename T>
+int apply_bc(mif_ctx* c, mif_field* const v[3], const FnDesc& f, double t, const PressureRim& rim = PressureRim{}) {
+  void* F[3] = {v[0]->data, v[1]->data, v[2]->data};
+  KTimer tm(c, MIF_KC_BC);
+  launch_bc<T>(c->g, c->L, F, f, t, c->stream, rim);
+  return MIF_OK;
+}
+
+// Stage st and the boundary values of its output O1, f at time t.
 // phi (not null): the previous stage's projection fused in, with time step
 // pdts and the increment's mean c->phi_mean; the incremented pressure goes to
-// pout, here and on the points the stage's tiles leave out: by the boundary
-// pass that follows (rim, for apply_bc), or by a pass of its own (rim null).
+// pout, also on the points the stage's tiles leave out (PressureRim).
+// Boundary values and rim are written by the stage kernel's launch where it
+// can (stage_shell), else by a boundary pass.
 template <typename T>
 int stage(mif_ctx* c, int st, mif_field* const X[3], mif_field* const A[3], mif_field* const O1[3],
-          mif_field* const O2[3], const void* p, double a1, double a2, double b, const void* phi = nullptr,
-          double pdts = 0, void* pout = nullptr, PressureRim* rim = nullptr) {
+          mif_field* const O2[3], const FnDesc& f, double t, const void* p, double a1, double a2, double b,
+          const void* phi = nullptr, double pdts = 0, void* pout = nullptr) {
   StageArgs s{};
   for (int q = 0; q < 3; q++) {
     s.X[q] = X[q]->data;
@@ -659,27 +669,15 @@ int stage(mif_ctx* c, int st, mif_field* const X[3], mif_field* const A[3], mif_
   s.pdts = pdts;
   s.pmean = phi ? c->phi_mean : nullptr;
   s.pout = pout;
+  PressureRim rim;
+  if (phi) rim = PressureRim{p, phi, pout, c->phi_mean};
+  const StageShell sh = stage_shell(c->g, c->L, true, s.O1, f, t, rim);
   {
-    KTimer t(c, MIF_KC_STAGE);
-    launch_stage<T>(st, c->g, c->L, s, c->stream);
+    KTimer tm(c, MIF_KC_STAGE);
+    launch_stage<T>(st, c->g, c->L, s, sh, c->stream);
   }
-  if (phi && rim) {
-    *rim = PressureRim{p, phi, pout, c->phi_mean};
-  } else if (phi) {
-    KTimer t(c, MIF_KC_PRESSURE_RIM);
-    launch_p_rim<T>(c->g, c->L, (const T*)p, (const T*)phi, (T*)pout, c->phi_mean, c->stream);
-  }
+  if (!sh.on) apply_bc<T>(c, O1, f, t, rim);
   if (phi) c->phi_mean = nullptr;
-  return MIF_OK;
-}
-
-// rim: the pressure rim of the fused stage kernel just launched, written in
-// the same launch
-template <typename T>
-int apply_bc(mif_ctx* c, mif_field* const v[3], const FnDesc& f, double t, const PressureRim& rim = PressureRim{}) {
-  void* F[3] = {v[0]->data, v[1]->data, v[2]->data};
-  KTimer tm(c, MIF_KC_BC);
-  launch_bc<T>(c->g, c->L, F, f, t, c->stream, rim);
   return MIF_OK;
 }
 
@@ -764,51 +762,48 @@ int full_timestep(mif_ctx* c, mif_field* const vel[3], mif_field* const buf[3], 
     c->sweeps = sweeps;
     return r;
   };
-  // the pressure rim of each fused stage kernel is written by the boundary
-  // pass that follows it (one launch)
-  PressureRim rim;
   // Stage 1 (src/Timestep.cpp:107-117), with the previous step's last
   // projection when a multi-step call left it pending
   {
     const double a1 = 64.0 / 120.0 * dt;
     if (fuse && cs.pending_dts > 0) {
-      rc = stage<T>(c, 1, vel, nullptr, buf, buf2, pin(), a1, 0.0, a1, pb->data, cs.pending_dts, pnext(), &rim);
+      rc = stage<T>(c, 1, vel, nullptr, buf, buf2, ev[0], st.time[1], pin(), a1, 0.0, a1, pb->data, cs.pending_dts,
+                    pnext());
       cs.cur ^= 1;
       cs.pending_dts = 0;
     } else {
-      rc = stage<T>(c, 1, vel, nullptr, buf, buf2, pin(), a1, 0.0, a1);
+      rc = stage<T>(c, 1, vel, nullptr, buf, buf2, ev[0], st.time[1], pin(), a1, 0.0, a1);
     }
     if (rc) return rc;
   }
-  apply_bc<T>(c, buf, ev[0], st.time[1], rim);
   if ((rc = solve(1, buf))) return rc;
   if (!fuse) project<T>(c, buf, p, pb, st.dt_s[1]);
   // Stage 2 (src/Timestep.cpp:119-129)
   {
     const double a1 = -34.0 / 120.0 * dt, a2 = 50.0 / 120.0 * dt;
     if (fuse) {
-      rc = stage<T>(c, 2, buf, buf2, buf2, vel, pin(), a1, a2, a1 + a2, pb->data, st.dt_s[1], pnext(), &rim);
+      rc = stage<T>(c, 2, buf, buf2, buf2, vel, ev[1], st.time[2], pin(), a1, a2, a1 + a2, pb->data, st.dt_s[1],
+                    pnext());
       cs.cur ^= 1;
     } else {
-      rc = stage<T>(c, 2, buf, buf2, buf2, vel, pin(), a1, a2, a1 + a2);
+      rc = stage<T>(c, 2, buf, buf2, buf2, vel, ev[1], st.time[2], pin(), a1, a2, a1 + a2);
     }
     if (rc) return rc;
   }
-  apply_bc<T>(c, buf2, ev[1], st.time[2], rim);
   if ((rc = solve(2, buf2))) return rc;
   if (!fuse) project<T>(c, buf2, p, pb, st.dt_s[2]);
   // Stage 3 (src/Timestep.cpp:131-140)
   {
     const double a2 = -50.0 / 120.0 * dt, a3 = 90.0 / 120.0 * dt;
     if (fuse) {
-      rc = stage<T>(c, 3, buf2, vel, vel, nullptr, pin(), 0.0, a3, a2 + a3, pb->data, st.dt_s[2], pnext(), &rim);
+      rc = stage<T>(c, 3, buf2, vel, vel, nullptr, ev[2], st.time[3], pin(), 0.0, a3, a2 + a3, pb->data, st.dt_s[2],
+                    pnext());
       cs.cur ^= 1;
     } else {
-      rc = stage<T>(c, 3, buf2, vel, vel, nullptr, pin(), 0.0, a3, a2 + a3);
+      rc = stage<T>(c, 3, buf2, vel, vel, nullptr, ev[2], st.time[3], pin(), 0.0, a3, a2 + a3);
     }
     if (rc) return rc;
   }
-  apply_bc<T>(c, vel, ev[2], st.time[3], rim);
   if ((rc = solve(3, vel))) return rc;
   if (fuse && !last) {
     cs.pending_dts = st.dt_s[3];
@@ -837,27 +832,24 @@ int velocity_timestep(mif_ctx* c, mif_field* const vel[3], mif_field* const buf[
     s.R[q] = rhs[q]->data;
     s.B[q] = buf[q]->data;
   }
-  for (int q = 0; q < 3; q++) s.X[q] = vel[q]->data;
-  s.t = t_n;
-  {
-    KTimer t(c, MIF_KC_STAGE);
-    launch_vel_stage<T>(1, c->g, c->L, s, c->stream);
-  }
-  apply_bc<T>(c, buf, ev[0], time_1);
-  for (int q = 0; q < 3; q++) s.X[q] = buf[q]->data;
-  s.t = time_1;
-  {
-    KTimer t(c, MIF_KC_STAGE);
-    launch_vel_stage<T>(2, c->g, c->L, s, c->stream);
-  }
-  apply_bc<T>(c, vel, ev[1], time_2);
-  for (int q = 0; q < 3; q++) s.X[q] = vel[q]->data;
-  s.t = time_2;
-  {
-    KTimer t(c, MIF_KC_STAGE);
-    launch_vel_stage<T>(3, c->g, c->L, s, c->stream);
-  }
-  apply_bc<T>(c, buf, ev[2], final_time);
+  // stage n from X at time t, its output out with the boundary values at t_bc
+  auto run = [&](int n, mif_field* const X[3], double t, mif_field* const out[3], double t_bc) {
+    void* F[3];
+    for (int q = 0; q < 3; q++) {
+      s.X[q] = X[q]->data;
+      F[q] = out[q]->data;
+    }
+    s.t = t;
+    const StageShell sh = stage_shell(c->g, c->L, false, F, ev[n - 1], t_bc, PressureRim{});
+    {
+      KTimer tm(c, MIF_KC_STAGE);
+      launch_vel_stage<T>(n, c->g, c->L, s, sh, c->stream);
+    }
+    if (!sh.on) apply_bc<T>(c, out, ev[n - 1], t_bc);
+  };
+  run(1, vel, t_n, buf, time_1);
+  run(2, buf, time_1, vel, time_2);
+  run(3, vel, time_2, buf, final_time);
   // velocity.swap_data(velocity_buffer) (src/TimestepVelocity.cpp:89)
   for (int q = 0; q < 3; q++) std::swap(vel[q]->data, buf[q]->data);
   LAUNCHCHK(c);

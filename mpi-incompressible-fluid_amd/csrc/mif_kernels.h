@@ -131,23 +131,50 @@ struct FusedIO {
   const Red3* bmean = nullptr;
 };
 
-template <typename T>
-void launch_stage(int stage, const DGrid& g, const Layout& L, const StageArgs& s, hipStream_t st);
 // pout = pin + (phi - mean) on the pressure points a stage kernel with a fused
-// projection leaves out (outside the union of the components' interiors):
-// on its own (launch_p_rim) or in the boundary pass that follows the stage
-// (launch_bc with a PressureRim)
+// projection leaves out (outside the union of the components' interiors).
 struct PressureRim {
   const void* pin = nullptr;  // null: no rim
   const void* phi = nullptr;
   void* pout = nullptr;
   const Red3* mean = nullptr;
 };
+// The extents of the stage kernels' tiles (the union of the components'
+// interiors) and the rim's point counts per group.
+struct RimShape {
+  int imax, jmax, kmax;
+  long count[3];
+};
+struct BCArgs {
+  void* F[3];
+  FnDesc f;
+  double t;
+  double tf;        // time_factor (BC_ES, BC_VT)
+  int count[3][3];  // threads (opposite shell points) per (component, face pair)
+};
+// The boundary pass and the pressure rim of a stage, in the stage's own
+// launch: the stage kernel stores its boundary-adjacent points at their
+// periodic images too, and `rows` + 3 rows of nbx further workgroups fill the
+// wall faces and the rim.
+struct StageShell {
+  int on = 0;    // 0: a boundary pass follows the stage
+  int nbx = 0;   // workgroups of a row
+  int rows = 0;  // (wall axis, component) rows; the rim's three come after them
+  BCArgs a{};
+  PressureRim rim{};
+  RimShape rs{};
+};
+// The shell of a stage (of the full or the velocity-only step) that writes F,
+// whose boundary data are f at time t.
+StageShell stage_shell(const DGrid& g, const Layout& L, bool full_step, void* const F[3], const FnDesc& f, double t,
+                       const PressureRim& rim);
+
 template <typename T>
-void launch_p_rim(const DGrid& g, const Layout& L, const T* pin, const T* phi, T* pout, const Red3* mean,
+void launch_stage(int stage, const DGrid& g, const Layout& L, const StageArgs& s, const StageShell& sh,
                   hipStream_t st);
 template <typename T>
-void launch_vel_stage(int stage, const DGrid& g, const Layout& L, const VelStageArgs& s, hipStream_t st);
+void launch_vel_stage(int stage, const DGrid& g, const Layout& L, const VelStageArgs& s, const StageShell& sh,
+                      hipStream_t st);
 // Fills the axis tables (axis_index) of n indices per axis.
 void launch_axis_tables(const DGrid& g, double* tab, int n, hipStream_t st);
 template <typename T>

@@ -159,7 +159,16 @@ constexpr bool kStageVec = true;
 // the pressure gradient uses p + phi - mean, and that incremented pressure is
 // stored into pout at the tile's points (another buffer than p: neighbouring
 // threads and tiles read p).
-template <typename T, int KIND, bool FT = false, bool NT = false, bool VEC = false, bool PROJ = false>
+// SHELL: the boundary shell of the output is written in this launch
+// (StageShell), by workgroups beyond the tiles' and (2: some axis is periodic)
+// by the threads of the points that have periodic images.
+template <typename T>
+__device__ inline void shell_block(const DGrid& g, const Layout& L, const StageShell& sh, int b, int t);
+struct NoShell {};
+template <int SHELL>
+using ShellArg = std::conditional_t<(SHELL > 0), StageShell, NoShell>;
+
+template <typename T, int KIND, bool FT = false, bool NT = false, bool VEC = false, bool PROJ = false, int SHELL = 0>
 // (FP64 full step: at most 80 VGPRs, i.e. three 512-thread workgroups per CU;
 // with the fused projection 128, two workgroups, which its LDS allows anyway;
 // FP32 with the fused projection, and the FP32 velocity-only kinds with the
@@ -169,8 +178,10 @@ template <typename T, int KIND, bool FT = false, bool NT = false, bool VEC = fal
 __global__ void __launch_bounds__(512)
 __attribute__((amdgpu_waves_per_eu(KIND <= 3 && (sizeof(T) == 8 || PROJ) ? (sizeof(T) == 8 && PROJ ? 4 : 6)
                                                                       : (FT && sizeof(T) == 4 ? 6 : 1))))
-k_stage(DGrid g, Layout L, StageArgs s, VelStageArgs vs, int imax, int jmax, int kmax, int ntx, int nty, int ntiles, int kchunk) {
+k_stage(DGrid g, Layout L, StageArgs s, VelStageArgs vs, ShellArg<SHELL> sh, int imax, int jmax, int kmax, int ntx, int nty,
+        int ntiles, int kchunk) {
   static_assert(!PROJ || KIND <= 3, "a fused projection belongs to the full-step kinds");
+  static_assert(SHELL < 2 || KIND <= 3, "images are stored by the full-step kinds");
   // ring slots: 3 (planes k-1, k, k+1; two barriers per plane) or 4 and
   // more (plane k+2 is committed into a free slot while plane k is
   // computed; one barrier per plane)
@@ -190,6 +201,12 @@ k_stage(DGrid g, Layout L, StageArgs s, VelStageArgs vs, int imax, int jmax, int
   constexpr int NSP = 4, PHX = SHX + 1, PHE = (SHY + 1) * PHX, PHQ = (PHE + STN - 1) / STN;
   __shared__ T phl[PL ? NSP : 1][PL ? PHE : 1];
   const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * STX + tx;
+  if constexpr (SHELL > 0) {
+    if ((int)blockIdx.x >= ntiles) {
+      shell_block<T>(g, L, sh, blockIdx.x - ntiles, tid);
+      return;
+    }
+  }
   const int tile = xcd_tile(blockIdx.x, ntiles);
   const int bx = tile % ntx, by = (tile / ntx) % nty, bz = tile / (ntx * nty);
   const int i0 = bx * STX + 1, j0 = by * STY + 1, k0 = bz * kchunk + 1;
@@ -436,8 +453,35 @@ k_stage(DGrid g, Layout L, StageArgs s, VelStageArgs vs, int imax, int jmax, int
   // and i <= imax, j <= jmax, k <= kmax) and their values are not used, so
   // the number of loads in flight is fixed for the compiler's waits.
   const long oc = L.idx(min(i, imax), min(j, jmax), 0);
+  // columns with periodic images in some component's field
+  const bool edge_ij = SHELL == 2 && ((g.periodic[0] && (i == 1 || i == g.N[0] - 2)) ||
+                                 (g.periodic[1] && (j == 1 || j == g.N[1] - 2 || j == g.N[1] - 1)));
   for (int k = k0; k < k1; k++) {
     const long o = L.idx(i, j, k);
+    const bool edge = edge_ij || (SHELL == 2 && g.periodic[2] && (k == 1 || k >= g.N[2] - 2));
+    // the value of interior point (i, j, k) of component c at its periodic
+    // images (one per axis at most: stage_shell asks for four points)
+    auto images = [&](int c, void* F, T v) {
+      // the column opaque to the compiler, which would keep every address of
+      // this branch in registers over the loop (28 VGPRs) otherwise
+      int ii = i, jj = j;
+      asm volatile("" : "+v"(ii), "+v"(jj));
+      int e[3];
+      extents(g, c, e);
+      auto image = [&](int ax, int q) { return g.periodic[ax] ? (q == 1 ? e[ax] - 1 : (q == e[ax] - 2 ? 0 : -1)) : -1; };
+      const int xi = image(0, ii), yi = image(1, jj), zi = image(2, k);
+      auto row = [&](int jr, int kr) {
+        T* r = (T*)F + L.idx(0, jr, kr);
+        if (jr != jj || kr != k) r[ii] = v;
+        if (xi >= 0) r[xi] = v;
+      };
+      row(jj, k);
+      if (yi >= 0) row(yi, k);
+      if (zi >= 0) {
+        row(jj, zi);
+        if (yi >= 0) row(yi, zi);
+      }
+    };
     const long ol = oc + (long)k * L.plane;
     T p0 = (T)0, pm[3] = {(T)0, (T)0, (T)0}, av[3] = {(T)0, (T)0, (T)0}, bv[3] = {(T)0, (T)0, (T)0};
     T f0 = (T)0, fm[3] = {(T)0, (T)0, (T)0};  // fused projection: phi at the point and below it
@@ -533,10 +577,15 @@ k_stage(DGrid g, Layout L, StageArgs s, VelStageArgs vs, int imax, int jmax, int
             // point outside component c's interior is a boundary-shell
             // point, which the boundary pass rewrites after the stage (O1)
             // or nothing reads (O2); threads outside the tile store at the
-            // shell point (0, 0, k)
-            const long os = in_tile ? o : L.idx(0, 0, k);
+            // shell point (0, 0, k).  SHELL: the shell is written by this
+            // launch, and both store into the padding beyond the component's
+            // extents (row N1 of u and w, column N0 of v)
+            long os = in_tile ? o : L.idx(0, 0, k);
+            if constexpr (SHELL > 0) os = inside[c] ? o : (c == 1 ? L.idx(g.N[0], 0, k) : L.idx(0, g.N[1], k));
             store_out<NT>(&((T*)s.O1[c])[os], o1);
             if constexpr (KIND <= 2) store_out<NT>(&((T*)s.O2[c])[os], o2);
+            if constexpr (SHELL == 2)
+              if (edge && inside[c]) images(c, s.O1[c], o1);
           } else {
             store_out<NT>(&((T*)s.O1[c])[o], o1);
             if constexpr (KIND <= 2) store_out<NT>(&((T*)s.O2[c])[o], o2);
@@ -554,15 +603,17 @@ k_stage(DGrid g, Layout L, StageArgs s, VelStageArgs vs, int imax, int jmax, int
             fc = eval_at(g, vs.forcing, c, c, vs.t, i, j, k);
           }
           const T f = rhs + (T)fc;
+          T o1;
           if constexpr (KIND == 4) {
             store_out<NT>(&((T*)vs.R[c])[o], f);
-            store_out<NT>(&((T*)vs.B[c])[o], x + dt * (T)(8.0 / 15.0) * f);
+            o1 = x + dt * (T)(8.0 / 15.0) * f;
           } else if constexpr (KIND == 5) {
             store_out<NT>(&((T*)vs.R[c])[o], bv[c] + dt * ((T)(1.0 / 4.0) * av[c]));
-            store_out<NT>(&((T*)vs.V[c])[o], bv[c] + dt * ((T)(1.0 / 4.0) * av[c] + (T)(5.0 / 12.0) * f));
+            o1 = bv[c] + dt * ((T)(1.0 / 4.0) * av[c] + (T)(5.0 / 12.0) * f);
           } else {
-            store_out<NT>(&((T*)vs.B[c])[o], av[c] + dt * ((T)(3.0 / 4.0) * f));
+            o1 = av[c] + dt * ((T)(3.0 / 4.0) * f);
           }
+          store_out<NT>(&((T*)(KIND == 5 ? vs.V[c] : vs.B[c]))[o], o1);
         }
       }
       if constexpr (PROJ) {
@@ -602,12 +653,6 @@ k_stage(DGrid g, Layout L, StageArgs s, VelStageArgs vs, int imax, int jmax, int
 __host__ __device__ inline int rim_out_count(int n, int mx) { return 1 + max(0, n - 1 - mx); }
 __device__ inline int rim_out_index(int t, int mx) { return t == 0 ? 0 : mx + t; }
 
-// The extents of the stage kernels' tiles (the union of the components'
-// interiors) and the rim's point counts per group.
-struct RimShape {
-  int imax, jmax, kmax;
-  long count[3];
-};
 inline RimShape rim_shape(const DGrid& g) {
   int eu[3], ev[3], ew[3];
   extents(g, 0, eu);
@@ -656,14 +701,6 @@ __device__ inline void p_rim_point(const DGrid& g, const Layout& L, int grp, lon
   pout[o] = pin[o] + (phi[o] - mv);
 }
 
-template <typename T>
-__global__ void __launch_bounds__(256) k_p_rim(DGrid g, Layout L, const T* __restrict__ pin, const T* __restrict__ phi,
-                                               T* __restrict__ pout, const Red3* __restrict__ mean, int imax, int jmax,
-                                               int kmax) {
-  p_rim_point<T>(g, L, blockIdx.y, (long)blockIdx.x * blockDim.x + threadIdx.x, pin, phi, pout, mean, imax, jmax,
-                 kmax);
-}
-
 // Boundary value of component c at point (i, j, k) of a face; ev(s, c, i, j, k)
 // is component c of the exact velocity at the point of staggering s.
 template <typename Ev>
@@ -693,14 +730,6 @@ __device__ inline double face_value(const DGrid& g, Ev ev, int c, int face, int 
   const double dw_dz = (ev(2, 2, in, j, k + 1) - ev(2, 2, in, j, k)) * g.one_over_h[2];
   return hi ? ub - g.h_over_2[0] * (dv_dy + dw_dz) : ub + g.h_over_2[0] * (dv_dy + dw_dz);
 }
-
-struct BCArgs {
-  void* F[3];
-  FnDesc f;
-  double t;
-  double tf;        // time_factor (BC_ES, BC_VT)
-  int count[3][3];  // threads (opposite shell points) per (component, face pair)
-};
 
 // Face data of a boundary pass: BC_ZERO homogeneous data (no-slip walls),
 // every face value is 0 and the function evaluation code is compiled out,
@@ -773,6 +802,49 @@ __device__ inline T shell_value(const DGrid& g, const Layout& L, const BCArgs& a
           c, face, s[0], s[1], s[2]);
   }
   return F[L.idx(s[0], s[1], s[2])];
+}
+
+// Workgroup b of a stage's shell (StageShell), thread t of 512: two opposite
+// wall points, or a point of the pressure rim.  The points of wall axis z are
+// whole planes (ghosts of periodic axes included); those of y and x leave out
+// the wall planes that z, then y have.
+template <typename T>
+__device__ inline void shell_block(const DGrid& g, const Layout& L, const StageShell& sh, int b, int t) {
+  const int row = b / sh.nbx;
+  const long q = (long)(b - row * sh.nbx) * 512 + t;
+  if (row >= sh.rows) {
+    p_rim_point<T>(g, L, row - sh.rows, q, (const T*)sh.rim.pin, (const T*)sh.rim.phi, (T*)sh.rim.pout, sh.rim.mean,
+                   sh.rs.imax, sh.rs.jmax, sh.rs.kmax);
+    return;
+  }
+  const int c = row % 3;
+  int wall = row / 3, axis = 2;
+  for (int a = 2; a >= 0; a--)
+    if (!g.periodic[a] && wall-- == 0) axis = a;
+  int e[3];
+  extents(g, c, e);
+  // the two other axes: ranges [lo, lo + n)
+  const int a0 = axis == 0 ? 1 : 0, a1 = axis == 2 ? 1 : 2;
+  const int lo0 = a0 > axis && !g.periodic[a0] ? 1 : 0, lo1 = a1 > axis && !g.periodic[a1] ? 1 : 0;
+  const int n0 = e[a0] - 2 * lo0, n1 = e[a1] - 2 * lo1;
+  if (q >= (long)n0 * n1) return;
+  const int q0 = lo0 + (int)(q % n0), q1 = lo1 + (int)(q / n0);
+  T* F = (T*)sh.a.F[c];
+#pragma unroll 1
+  for (int side = 0; side < 2; side++) {
+    const int w = side ? e[axis] - 1 : 0;
+    const int i = axis == 0 ? w : q0, j = axis == 1 ? w : (axis == 0 ? q0 : q1), k = axis == 2 ? w : q1;
+    T v;
+    if (sh.a.f.kind == MIF_FN_ZERO)
+      v = (T)0;
+    else if (sh.a.f.kind == MIF_FN_ES_VELOCITY)
+      v = shell_value<T, BC_ES>(g, L, sh.a, c, e, i, j, k, F);
+    else if (sh.a.f.kind == MIF_FN_VT_VELOCITY)
+      v = shell_value<T, BC_VT>(g, L, sh.a, c, e, i, j, k, F);
+    else
+      v = shell_value<T, BC_LID>(g, L, sh.a, c, e, i, j, k, F);
+    F[L.idx(i, j, k)] = v;
+  }
 }
 
 // Each thread owns the two opposite shell points of one (pair, position):
@@ -1223,7 +1295,7 @@ static int stage_chunk(long cols, int planes, int most) {
 
 template <typename T, int KIND, bool FT = false, bool NT = false>
 static void launch_stage_kind(const DGrid& g, const Layout& L, const StageArgs& s, const VelStageArgs& vs,
-                              hipStream_t st) {
+                              const StageShell& sh, hipStream_t st) {
   // union of the three components' interiors
   int eu[3], ev[3], ew[3];
   extents(g, 0, eu);
@@ -1235,11 +1307,22 @@ static void launch_stage_kind(const DGrid& g, const Layout& L, const StageArgs& 
   constexpr int STX = StageTile<T>::STX, STY = StageTile<T>::STY;
   const int ntx = (imax + STX - 1) / STX, nty = (jmax + STY - 1) / STY;
   const dim3 blk(STX, STY, 1);
-  auto go = [&](auto vec, auto proj) {
+  auto run = [&](auto vec, auto proj, auto shell) {
     constexpr bool V = decltype(vec)::value, P = decltype(proj)::value;
+    constexpr int S = decltype(shell)::value;
     const int kchunk = stage_chunk(ntx * nty, kmax, stage_planes<T, KIND, NT, P>());
     const int ntiles = ntx * nty * ((kmax + kchunk - 1) / kchunk);
-    k_stage<T, KIND, FT, NT, V, P><<<ntiles, blk, 0, st>>>(g, L, s, vs, imax, jmax, kmax, ntx, nty, ntiles, kchunk);
+    const int nshell = S > 0 ? sh.nbx * (sh.rows + (sh.rim.pin ? 3 : 0)) : 0;
+    ShellArg<S> arg;
+    if constexpr (S > 0) arg = sh;
+    k_stage<T, KIND, FT, NT, V, P, S><<<ntiles + nshell, blk, 0, st>>>(g, L, s, vs, arg, imax, jmax, kmax, ntx, nty,
+                                                                      ntiles, kchunk);
+  };
+  auto go = [&](auto vec, auto proj) {
+    if (!sh.on) return run(vec, proj, std::integral_constant<int, 0>{});
+    if (!g.periodic[0] && !g.periodic[1] && !g.periodic[2]) return run(vec, proj, std::integral_constant<int, 1>{});
+    // stage_shell: full step, small grids
+    if constexpr (!NT && KIND <= 3) run(vec, proj, std::integral_constant<int, 2>{});
   };
   using yes = std::true_type;
   using no = std::false_type;
@@ -1272,33 +1355,63 @@ static void launch_stage_kind(const DGrid& g, const Layout& L, const StageArgs& 
   go(no{}, no{});
 }
 
-// ---------------------------------------------------------------------------
-// The pressure increment of a projection fused into the next stage
-// (update_pressure, src/Timestep.cpp:76-81: p += phi at every point), on the
-// points the stage kernel's tiles leave out: those of the pressure's extents
-// outside [1, imax] x [1, jmax] x [1, kmax] (imax, jmax, kmax: the union of
-// the velocity components' interiors).  pout = pin + (phi - mean).
-// Three groups of points: the k planes outside [1, kmax]; within it the j
-// rows outside [1, jmax]; within both the i columns outside [1, imax].
-// ---------------------------------------------------------------------------
-template <typename T>
-void launch_p_rim(const DGrid& g, const Layout& L, const T* pin, const T* phi, T* pout, const Red3* mean,
-                  hipStream_t st) {
-  const RimShape rs = rim_shape(g);
-  const long mx = max(rs.count[0], max(rs.count[1], rs.count[2]));
-  k_p_rim<T><<<dim3((unsigned)((mx + 255) / 256), 3, 1), 256, 0, st>>>(g, L, pin, phi, pout, mean, rs.imax, rs.jmax,
-                                                                      rs.kmax);
+// The launch saved against what the stage kernel loses by it.  Without a
+// periodic axis the shell is workgroups of its own (step with the boundary
+// pass -> in the stage's launch; 33^3, 65^3, 129^3, 193^3, 257^3 nodes, us):
+// velocity-only FP64 33.8 -> 20.5, 45.0 -> 33, 154 -> 139, 559 -> 541, 1216 ->
+// 1205 (256^3), mixed 32.8 -> 22.0, 48.3 -> 36.3, 107.5 -> 94, 425 -> 413, 780
+// -> 770 (256^3); full step, Ethier-Steinman, FP64 123 -> 112, 160 -> 144, 448
+// -> 429, 1370 -> 1353, 2692 -> 2693, mixed 123 -> 110, 152 -> 136, 297 -> 284,
+// 826 -> 824, 1467 -> 1494: there up to kShellMaxElems.  With periodic axes
+// the plane loop stores images under branches, and the stage kernel is slower
+// (channel step, 33^3, 49^3, 65^3, 81^3, 129^3, us): FP64 122 -> 114, 131 ->
+// 126, 151 -> 146, 214 -> 221, 421 -> 429, mixed 119 -> 109, 128 -> 122, 146 ->
+// 139, 173 -> 178, 290 -> 299: up to kShellMaxPoints.
+constexpr long kShellMaxElems = 8L << 20;
+constexpr long kShellMaxPoints = 300000;
+
+StageShell stage_shell(const DGrid& g, const Layout& L, bool full_step, void* const F[3], const FnDesc& f, double t,
+                       const PressureRim& rim) {
+  StageShell sh;
+  if (f.kind != MIF_FN_ZERO && f.kind != MIF_FN_ES_VELOCITY && f.kind != MIF_FN_VT_VELOCITY &&
+      f.kind != MIF_FN_LID_1 && f.kind != MIF_FN_LID_2)
+    return sh;
+  bool images = false;
+  for (int a = 0; a < 3; a++) {
+    if (g.periodic[a] && g.N[a] < 4) return sh;  // two images of a point on one axis
+    images = images || g.periodic[a];
+  }
+  if (images ? !full_step || (long)g.N[0] * g.N[1] * g.N[2] > kShellMaxPoints : full_step && L.elems > kShellMaxElems)
+    return sh;
+  sh.on = 1;
+  long mx = 0;
+  for (int a = 0; a < 3; a++) {
+    if (g.periodic[a]) continue;
+    sh.rows += 3;
+    const int a0 = a == 0 ? 1 : 0, a1 = a == 2 ? 1 : 2;
+    mx = max(mx, (long)(g.N[a0] + 1) * (g.N[a1] + 1));
+  }
+  for (int c = 0; c < 3; c++) sh.a.F[c] = F[c];
+  sh.a.f = f;
+  sh.a.t = t;
+  if (f.kind == MIF_FN_ES_VELOCITY || f.kind == MIF_FN_VT_VELOCITY) sh.a.tf = time_factor(f.kind, t, f.Re);
+  sh.rim = rim;
+  sh.rs = rim_shape(g);
+  if (rim.pin) mx = max(mx, max(sh.rs.count[0], max(sh.rs.count[1], sh.rs.count[2])));
+  sh.nbx = (int)((mx + 511) / 512);
+  return sh;
 }
 
 template <typename T>
-void launch_stage(int stage, const DGrid& g, const Layout& L, const StageArgs& s, hipStream_t st) {
+void launch_stage(int stage, const DGrid& g, const Layout& L, const StageArgs& s, const StageShell& sh,
+                  hipStream_t st) {
   VelStageArgs vs{};
   if (stage == 1)
-    L.nt ? launch_stage_kind<T, 1, false, true>(g, L, s, vs, st) : launch_stage_kind<T, 1>(g, L, s, vs, st);
+    L.nt ? launch_stage_kind<T, 1, false, true>(g, L, s, vs, sh, st) : launch_stage_kind<T, 1>(g, L, s, vs, sh, st);
   else if (stage == 2)
-    L.nt ? launch_stage_kind<T, 2, false, true>(g, L, s, vs, st) : launch_stage_kind<T, 2>(g, L, s, vs, st);
+    L.nt ? launch_stage_kind<T, 2, false, true>(g, L, s, vs, sh, st) : launch_stage_kind<T, 2>(g, L, s, vs, sh, st);
   else
-    L.nt ? launch_stage_kind<T, 3, false, true>(g, L, s, vs, st) : launch_stage_kind<T, 3>(g, L, s, vs, st);
+    L.nt ? launch_stage_kind<T, 3, false, true>(g, L, s, vs, sh, st) : launch_stage_kind<T, 3>(g, L, s, vs, sh, st);
 }
 
 // The velocity-only kinds read 6 to 9 arrays and write 3 to 6, and are bound by
@@ -1312,16 +1425,17 @@ void launch_stage(int stage, const DGrid& g, const Layout& L, const StageArgs& s
 constexpr long kVelNtMinFieldBytes = 40L << 20;
 
 template <typename T>
-void launch_vel_stage(int stage, const DGrid& g, const Layout& L, const VelStageArgs& vs, hipStream_t st) {
+void launch_vel_stage(int stage, const DGrid& g, const Layout& L, const VelStageArgs& vs, const StageShell& sh,
+                      hipStream_t st) {
   StageArgs s{};
   auto go = [&](auto ft, auto nt) {
     constexpr bool F = decltype(ft)::value, N = decltype(nt)::value;
     if (stage == 1)
-      launch_stage_kind<T, 4, F, N>(g, L, s, vs, st);
+      launch_stage_kind<T, 4, F, N>(g, L, s, vs, sh, st);
     else if (stage == 2)
-      launch_stage_kind<T, 5, F, N>(g, L, s, vs, st);
+      launch_stage_kind<T, 5, F, N>(g, L, s, vs, sh, st);
     else
-      launch_stage_kind<T, 6, F, N>(g, L, s, vs, st);
+      launch_stage_kind<T, 6, F, N>(g, L, s, vs, sh, st);
   };
   using yes = std::true_type;
   using no = std::false_type;
@@ -1530,9 +1644,9 @@ void launch_gather(const Layout& L, const T* F, const int* ijk, long n, double* 
 }
 
 #define MIF_INSTANTIATE(T)                                                                                          \
-  template void launch_stage<T>(int, const DGrid&, const Layout&, const StageArgs&, hipStream_t);                   \
-  template void launch_p_rim<T>(const DGrid&, const Layout&, const T*, const T*, T*, const Red3*, hipStream_t);    \
-  template void launch_vel_stage<T>(int, const DGrid&, const Layout&, const VelStageArgs&, hipStream_t);            \
+  template void launch_stage<T>(int, const DGrid&, const Layout&, const StageArgs&, const StageShell&, hipStream_t); \
+  template void launch_vel_stage<T>(int, const DGrid&, const Layout&, const VelStageArgs&, const StageShell&,       \
+                                    hipStream_t);                                                                   \
   template void launch_bc<T>(const DGrid&, const Layout&, void* const*, const FnDesc&, double, hipStream_t,         \
                              const PressureRim&);                                                                   \
   template void launch_periodic<T>(const DGrid&, const Layout&, T*, int, hipStream_t);                              \
