@@ -13,7 +13,11 @@
 // (w_0 = 1, else 2), and the inverse runs the other way, x_j = a_j + b_j and
 // x_{R-j} = a_j - b_j with a from the even part (r_k or Y_{2q}) and b from
 // the odd part.  That is n multiply-adds per element and pass, on
-// V_MFMA_*_16X16X4 tiles: 16 lines by 16 coefficients, K = 4.
+// V_MFMA_*_16X16X4 tiles: 16 lines by 16 coefficients, K = 4.  A periodic line
+// of even length folds once more about n/4: with h = n/2, the terms of even
+// and odd k are sums over e_j + e_{h-j}, e_j - e_{h-j}, o_j - o_{h-j} and
+// o_j + o_{h-j} (j <= h/2), four parts of a quarter of the line each and n/2
+// multiply-adds per element (kQuadMin).
 //
 // Slot order, scaling, the fused divergence, unpack and defect passes are
 // those of mif_fft_pow2.hip.
@@ -29,12 +33,12 @@
 // rate) and the memory 60 us: the two phases of a workgroup overlap only
 // through the other three workgroups of its CU.
 //
-// Work split: a workgroup owns 16 lines; each wave owns one of the
-// H / 16 row tiles (H = R/2 + 1) of both matrices, for all lines (on x there
-// may be waves beyond those, launch_dense_pass).  The
-// folded lines (e and o) sit in LDS, the matrices are read fragment by
-// fragment from global memory (they are shared by all workgroups and stay in
-// L2; a fragment is one 16-byte load per lane in FP64).
+// Work split: a workgroup owns 16 lines; each wave owns one of the H / 16 row
+// tiles (H = R/2 + 1, or n/4 + 1) of every part's matrix, for all lines (on x
+// there may be waves beyond those, launch_dense_pass).  The folded lines sit
+// in LDS, the matrices are read fragment by fragment from global memory (they
+// are shared by all workgroups and stay in L2; a fragment is one 16-byte load
+// per lane in FP64).
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -86,7 +90,8 @@ enum { IO_PLAIN = 0, IO_FIELD = 1, IO_FIELD_DC = 2, IO_DEFECT = 3, IO_PACK = 4 }
 }  // namespace dense
 
 // MODE 0: forward, 1: inverse, 2: forward + scale + inverse (axis 2).
-template <typename T, int AXIS, int MODE, int IO, typename TV>
+// QUAD: four parts (a periodic line of even length), else two.
+template <typename T, int AXIS, int MODE, int IO, typename TV, bool QUAD>
 __global__ void __launch_bounds__(1024) k_dense(DGrid g, DensePlan P, const T* __restrict__ M, SpectralScale sc,
                                                T* __restrict__ B, long bp0, long bplane, FusedIO io) {
   using namespace dense;
@@ -94,11 +99,12 @@ __global__ void __launch_bounds__(1024) k_dense(DGrid g, DensePlan P, const T* _
   using Acc = typename Op::acc;
   using Frag = typename Op::frag;
   extern __shared__ __align__(16) unsigned char smem[];
-  const int H = P.H, KS = P.KS, KP = 8 * P.KS, n = P.n, R = P.R;
+  constexpr int NP = QUAD ? 4 : 2;
+  const int H = P.H, KS = P.KS, KP = 8 * P.KS, n = P.n, R = P.R, h = n >> 1;
   const bool periodic = P.periodic;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nthr = blockDim.x, W = nthr >> 6;
   const int n0 = g.npts[0], n1 = g.npts[1], n2 = g.npts[2];
-  // e and o: [row][line] on the strided axes, [line][row] on x
+  // the parts: [row][line] on the strided axes, [line][row] on x
   const int px = KP + Op::kPadX;
   const int half = AXIS == 0 ? NL * px : KP * NL;
   T* const Eo = (T*)smem;
@@ -114,14 +120,49 @@ __global__ void __launch_bounds__(1024) k_dense(DGrid g, DensePlan P, const T* _
   const long ms = AXIS == 0 ? 1 : (AXIS == 1 ? bp0 : bplane);
   // element j of the physical line and its mirror image; self: it has none
   auto self = [&](int j) -> bool { return 2 * j == R || (periodic && j == 0); };
-  // spectral slots of row r of the even and odd parts (-1: none)
-  auto slot_e = [&](int r) -> int {
-    const int s = periodic ? r : 2 * r;
-    return (periodic ? 2 * r <= n : s < n) ? s : -1;
+  // spectral slot of row r of part p (-1: none)
+  auto slot = [&](int p, int r) -> int {
+    if constexpr (QUAD) {
+      const int k = 2 * r + (p & 1);
+      if (p < 2) return k <= h ? k : -1;
+      return k >= 1 && k < h ? n - k : -1;
+    } else {
+      if (periodic) return p == 0 ? (2 * r <= n ? r : -1) : (r >= 1 && 2 * r < n ? n - r : -1);
+      return 2 * r + p < n ? 2 * r + p : -1;
+    }
   };
-  auto slot_o = [&](int r) -> int {
-    if (periodic) return r >= 1 && 2 * r < n ? n - r : -1;
-    return 2 * r + 1 < n ? 2 * r + 1 : -1;
+  // The parts of row j from its points: x_j and x_{R-j}; QUAD: x_j, x_{n-j},
+  // x_{h-j}, x_{h+j} (points that coincide come as zeros)
+  auto fold = [&](int j, const T (&x)[NP], T (&f)[NP]) {
+    if constexpr (QUAD) {
+      const bool mid = 2 * j == h;
+      const T e0 = x[0] + x[1], o0 = j == 0 ? (T)0 : x[0] - x[1], e1 = x[2] + x[3], o1 = j == 0 ? (T)0 : x[2] - x[3];
+      f[0] = e0 + e1;
+      f[1] = mid ? (T)0 : e0 - e1;
+      f[2] = mid ? (T)0 : o0 - o1;
+      f[3] = o0 + o1;
+    } else {
+      f[0] = x[0] + x[1];
+      f[1] = self(j) ? (T)0 : x[0] - x[1];
+    }
+  };
+  // whether point q of a row's NP points is one of its own, and its index
+  auto own = [&](int j, int q) -> bool {
+    if constexpr (QUAD) return q == 0 || (q == 1 ? j > 0 : 2 * j != h && (q == 2 || j > 0));
+    else return q == 0 || !self(j);
+  };
+  auto point = [&](int j, int q) -> int {
+    if constexpr (QUAD) return q == 0 ? j : (q == 1 ? n - j : (q == 2 ? h - j : h + j));
+    else return q == 0 ? j : R - j;
+  };
+  // the value at point q of row j from the parts of the inverse
+  auto unfold = [&](const T (&f)[NP], int q) -> T {
+    if constexpr (QUAD) {
+      const T a = q < 2 ? f[0] + f[1] : f[0] - f[1], b = q < 2 ? f[2] + f[3] : f[3] - f[2];
+      return q & 1 ? a - b : a + b;
+    } else {
+      return q ? f[0] - f[1] : f[0] + f[1];
+    }
   };
 
   // ---- load, folded
@@ -166,8 +207,8 @@ __global__ void __launch_bounds__(1024) k_dense(DGrid g, DensePlan P, const T* _
     const double rmean = IO == IO_DEFECT ? io.bmean->s1 / io.bmean->s2 : 0.0;
     const double ihx2 = 1.0 / (g.h[0] * g.h[0]), ihy2 = 1.0 / (g.h[1] * g.h[1]), ihz2 = 1.0 / (g.h[2] * g.h[2]);
     // the value of point m of line l (a line outside the grid reads row 0
-    // and is dropped by its caller)
-    auto value = [&](int l, int m) -> T {
+    // and is dropped by its caller); mine: the caller is the point's only one
+    auto value = [&](int l, int m, bool mine) -> T {
       const long b = lbase[l];
       if constexpr (IO == IO_PLAIN) {
         return B[(b >= 0 ? b : 0) + m];
@@ -192,7 +233,7 @@ __global__ void __launch_bounds__(1024) k_dense(DGrid g, DensePlan P, const T* _
         const double dw_dz = ((double)w[o + io.L.plane] - (double)w[o]) * g.one_over_h[2];
         const double bv = (du_dx + dv_dy + dw_dz) / io.dt;
         if constexpr (IO == IO_FIELD_DC) {
-          if (b >= 0) {
+          if (b >= 0 && mine) {
             io.b64[b + m] = bv;
             const double wgt = owner_weight(g, 0, m) * lwt[l];
             dc_s += wgt * bv;
@@ -205,28 +246,32 @@ __global__ void __launch_bounds__(1024) k_dense(DGrid g, DensePlan P, const T* _
     for (int q = t; q < NL * KP; q += nthr) {
       const int l = (q * rkp) >> 22, j = q - l * KP;
       const bool ok = lbase[l] >= 0;
-      T e = 0, o = 0;
+      T f[NP] = {};
       if (j < H) {
-        const T a = value(l, j);
-        if (self(j)) {
-          e = ok ? a : (T)0;
-        } else {
-          const T b = value(l, R - j);
-          e = ok ? a + b : (T)0;
-          o = ok ? a - b : (T)0;
+        T x[NP];
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+          const bool mine = own(j, p);
+          const T v = value(l, mine ? point(j, p) : j, mine);
+          x[p] = mine ? v : (T)0;
         }
+        fold(j, x, f);
       }
-      Eo[at(j, l)] = e;
-      Eo[half + at(j, l)] = o;
+#pragma unroll
+      for (int p = 0; p < NP; p++) Eo[p * half + at(j, l)] = ok ? f[p] : (T)0;
     }
   } else if constexpr (AXIS == 0) {
     for (int q = t; q < NL * KP; q += nthr) {
       const int l = (q * rkp) >> 22, r = q - l * KP;
       const long b = lbase[l];
-      const int se = slot_e(r), so = slot_o(r);
-      const T e = B[b >= 0 && se >= 0 ? b + se : 0], o = B[b >= 0 && so >= 0 ? b + so : 0];
-      Eo[at(r, l)] = b >= 0 && se >= 0 ? e : (T)0;
-      Eo[half + at(r, l)] = b >= 0 && so >= 0 ? o : (T)0;
+      T f[NP];
+#pragma unroll
+      for (int p = 0; p < NP; p++) {
+        const int s = slot(p, r);
+        f[p] = B[b >= 0 && s >= 0 ? b + s : 0];
+      }
+#pragma unroll
+      for (int p = 0; p < NP; p++) Eo[p * half + at(r, l)] = b >= 0 && slot(p, r) >= 0 ? f[p] : (T)0;
     }
   } else {
     const int l = t & (NL - 1), step = nthr / NL;
@@ -236,92 +281,97 @@ __global__ void __launch_bounds__(1024) k_dense(DGrid g, DensePlan P, const T* _
     // U rows in flight per thread, from always-valid addresses
     constexpr int U = 4;
     for (int q = t / NL; q < KP; q += U * step) {
-      T a[U], b[U];
+      T a[U][NP];
 #pragma unroll
       for (int u = 0; u < U; u++) {
-        const int r = q + u * step;
-        int s1, s2;
-        if (MODE == 1) {
-          s1 = slot_e(r);
-          s2 = slot_o(r);
-          s1 = s1 < 0 ? 0 : s1;
-          s2 = s2 < 0 ? 0 : s2;
-        } else {
-          s1 = r < H ? r : 0;
-          s2 = self(s1) ? s1 : R - s1;
+        const int r = q + u * step, j = r < H ? r : 0;
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+          const int s = MODE == 1 ? max(slot(p, r), 0) : (own(j, p) ? point(j, p) : j);
+          a[u][p] = src[s * ms];
         }
-        a[u] = src[s1 * ms];
-        b[u] = src[s2 * ms];
       }
 #pragma unroll
       for (int u = 0; u < U; u++) {
         const int r = q + u * step;
         if (r >= KP) break;
-        T e, o;
+        T f[NP];
         if (MODE == 1) {
-          e = ok && slot_e(r) >= 0 ? a[u] : (T)0;
-          o = ok && slot_o(r) >= 0 ? b[u] : (T)0;
+#pragma unroll
+          for (int p = 0; p < NP; p++) f[p] = ok && slot(p, r) >= 0 ? a[u][p] : (T)0;
         } else {
           const bool in = ok && r < H;
-          e = in ? (self(r) ? a[u] : a[u] + b[u]) : (T)0;
-          o = in && !self(r) ? a[u] - b[u] : (T)0;
+          T x[NP];
+#pragma unroll
+          for (int p = 0; p < NP; p++) x[p] = in && own(r, p) ? a[u][p] : (T)0;
+          fold(r, x, f);
         }
-        Eo[at(r, l)] = e;
-        Eo[half + at(r, l)] = o;
+#pragma unroll
+        for (int p = 0; p < NP; p++) Eo[p * half + at(r, l)] = f[p];
       }
     }
   }
   __syncthreads();
 
-  // ---- products: acc[.][.][0] even part, [1] odd part, each in two chains.
-  // FP64: one per K step of a fragment.  FP32 (kBlocked): every eight terms
-  // are summed from zero and added to alternating totals, so that the longest
-  // chain of roundings is 8 + H/16 terms: the solve's error on a line of
-  // 120-283 nodes is then that of the mixed-radix transform (2e-7; 3e-7 with
-  // the FP64 scheme)
-  Acc acc[2][2];
+  // ---- products: acc[part][chain].  Two parts: two chains each, FP64 one
+  // per K step of a fragment, FP32 (kBlocked) every eight terms summed from
+  // zero and added to alternating totals, so that the longest chain of
+  // roundings is 8 + H/16 terms: the solve's error on a line of 120-283 nodes
+  // is then that of the mixed-radix transform (2e-7; 3e-7 with the FP64
+  // scheme).  Four parts: their rows are half as long, one chain each.
+  constexpr int NC = QUAD ? 1 : 2;
+  Acc acc[NP][NC];
 #pragma unroll
-  for (int c = 0; c < 4; c++) acc[c >> 1][c & 1] = Acc{0, 0, 0, 0};
-  auto multiply = [&](const T* Me) {
-    const T* Mo = Me + (long)P.MT * KS * 128;
+  for (int p = 0; p < NP; p++)
 #pragma unroll
-    for (int c = 0; c < 4; c++) acc[c >> 1][c & 1] = Acc{0, 0, 0, 0};
-    const Frag* fe = (const Frag*)Me + (long)wave * KS * 64 + lane;
-    const Frag* fo = (const Frag*)Mo + (long)wave * KS * 64 + lane;
-    Frag ne = fe[0], no = fo[0];
+    for (int c = 0; c < NC; c++) acc[p][c] = Acc{0, 0, 0, 0};
+  auto multiply = [&](const T* Md) {
+#pragma unroll
+    for (int p = 0; p < NP; p++)
+#pragma unroll
+      for (int c = 0; c < NC; c++) acc[p][c] = Acc{0, 0, 0, 0};
+    const Frag* fr = (const Frag*)Md + (long)wave * KS * 64 + lane;
+    const long part = (long)P.MT * KS * 64;
+    Frag next[NP];
+#pragma unroll
+    for (int p = 0; p < NP; p++) next[p] = fr[p * part];
     auto step = [&](int s, int par) {
-      const Frag ce = ne, co = no;
+      Frag cur[NP];
       const int s1 = s + 1 < KS ? s + 1 : s;  // next fragments requested before this step's products
-      ne = fe[s1 * 64];
-      no = fo[s1 * 64];
-      T le[2], lo[2];
+#pragma unroll
+      for (int p = 0; p < NP; p++) {
+        cur[p] = next[p];
+        next[p] = fr[p * part + s1 * 64];
+      }
+      T ln[NP][2];
 #pragma unroll
       for (int h = 0; h < 2; h++) {
         const int o = at(8 * s + 4 * h + (lane >> 4), lane & 15);
-        le[h] = Eo[o];
-        lo[h] = Eo[half + o];
+#pragma unroll
+        for (int p = 0; p < NP; p++) ln[p][h] = Eo[p * half + o];
       }
       auto mul = [&](T f, T x, Acc c) { return AXIS == 0 ? Op::mma(x, f, c) : Op::mma(f, x, c); };
       if constexpr (Op::kBlocked) {
         const Acc z = {0, 0, 0, 0};
-        acc[0][par] += mul(ce[1], le[1], mul(ce[0], le[0], z));
-        acc[1][par] += mul(co[1], lo[1], mul(co[0], lo[0], z));
+#pragma unroll
+        for (int p = 0; p < NP; p++)
+          acc[p][QUAD ? 0 : par] += mul(cur[p][1], ln[p][1], mul(cur[p][0], ln[p][0], z));
       } else {
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-          acc[0][h] = mul(ce[h], le[h], acc[0][h]);
-          acc[1][h] = mul(co[h], lo[h], acc[1][h]);
-        }
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+          for (int p = 0; p < NP; p++) acc[p][QUAD ? 0 : h] = mul(cur[p][h], ln[p][h], acc[p][QUAD ? 0 : h]);
       }
     };
     for (int s = 0; s < KS; s += 2) {
       step(s, 0);
       if (s + 1 < KS) step(s + 1, 1);
     }
-    acc[0][0] += acc[0][1];
-    acc[1][0] += acc[1][1];
+    if constexpr (NC == 2)
+#pragma unroll
+      for (int p = 0; p < NP; p++) acc[p][0] += acc[p][NC - 1];
   };
-  const long msize = 2L * P.MT * KS * 128;  // one direction's two matrices
+  const long msize = (long)NP * P.MT * KS * 128;  // one direction's matrices
   // the x passes may have waves without a row tile: they load and store only
   if (AXIS != 0 || wave < P.MT) multiply(M + (MODE == 1 ? msize : 0));
 
@@ -335,15 +385,17 @@ __global__ void __launch_bounds__(1024) k_dense(DGrid g, DensePlan P, const T* _
     for (int r = 0; r < 4; r++) {
       const int k = 16 * wave + Op::row(r, lane);
       if (k >= KP) continue;
-      const int se = slot_e(k), so = slot_o(k);
-      T e = 0, o = 0;
-      if (se >= 0) {
-        const double s = i == 0 && by == 0 && se == 0 ? 0.0 : (1.0 / (lxy + sc.lam[2][se])) * sc.inv_norm;
-        e = acc[0][0][r] * (T)s;
+#pragma unroll
+      for (int p = 0; p < NP; p++) {
+        const int sl = slot(p, k);
+        T x = 0;
+        if (sl >= 0) {
+          const double s =
+              p == 0 && i == 0 && by == 0 && sl == 0 ? 0.0 : (1.0 / (lxy + sc.lam[2][sl])) * sc.inv_norm;
+          x = acc[p][0][r] * (T)s;
+        }
+        Eo[p * half + at(k, l)] = x;
       }
-      if (so >= 0) o = acc[1][0][r] * (T)((1.0 / (lxy + sc.lam[2][so])) * sc.inv_norm);
-      Eo[at(k, l)] = e;
-      Eo[half + at(k, l)] = o;
     }
     __syncthreads();
     multiply(M + msize);
@@ -357,38 +409,44 @@ __global__ void __launch_bounds__(1024) k_dense(DGrid g, DensePlan P, const T* _
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         const int k = 16 * wave + Op::row(r, lane);
-        const T a = acc[0][0][r], b = acc[1][0][r];
-        if (MODE == 0) {
-          const int se = slot_e(k), so = slot_o(k);
-          if (se >= 0) dst[se * ms] = a;
-          if (so >= 0) dst[so * ms] = b;
-        } else if (k < H) {
-          dst[k * ms] = a + b;
-          if (!self(k)) dst[(R - k) * ms] = a - b;
+        T f[NP];
+#pragma unroll
+        for (int p = 0; p < NP; p++) f[p] = acc[p][0][r];
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+          if (MODE == 0) {
+            const int sl = slot(p, k);
+            if (sl >= 0) dst[sl * ms] = f[p];
+          } else if (k < H && own(k, p)) {
+            dst[point(k, p) * ms] = unfold(f, p);
+          }
         }
       }
     }
   } else {
     // lines back to LDS, so that whole rows are stored
-    const int pl = 2 * px;
+    const int pl = NP * px;
     __syncthreads();
     const int k = 16 * wave + (lane & 15);
-    const int se = slot_e(k), so = slot_o(k);
 #pragma unroll
     for (int r = 0; r < 4; r++) {
       T* x = Eo + Op::row(r, lane) * pl;
-      const T a = acc[0][0][r], b = acc[1][0][r];
-      if (MODE == 0) {
-        if (se >= 0) x[se] = a;
-        if (so >= 0) x[so] = b;
-      } else if (k < H) {
-        x[k] = a + b;
-        if (!self(k)) x[R - k] = a - b;
+      T f[NP];
+#pragma unroll
+      for (int p = 0; p < NP; p++) f[p] = acc[p][0][r];
+#pragma unroll
+      for (int p = 0; p < NP; p++) {
+        if (MODE == 0) {
+          const int sl = slot(p, k);
+          if (sl >= 0) x[sl] = f[p];
+        } else if (k < H && own(k, p)) {
+          x[point(k, p)] = unfold(f, p);
+        }
       }
     }
     __syncthreads();
     // a group of 2^lg lanes stores one line
-    const int lg = H <= 16 ? 4 : (H <= 32 ? 5 : 6);
+    const int lg = n <= 32 ? 4 : (n <= 64 ? 5 : 6);
     const int m0 = t & ((1 << lg) - 1);
     for (int l = t >> lg; l < NL; l += nthr >> lg) {
       const long b = lbase[l];
@@ -448,24 +506,41 @@ __global__ void __launch_bounds__(1024) k_dense(DGrid g, DensePlan P, const T* _
 // ---------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------
+// Periodic lines of even length from which four parts pay: half the products,
+// but half the row tiles too, and shorter ones leave the matrix cores waiting
+// for loads either way.  Two -> four parts (divergence / unpack / y / z pass,
+// us): FP64 78^3 points 9.8 / 9.2 / 8.0 / 11.7 -> 10.6 / 9.9 / 8.8 / 14.0, 102^3
+// 15.0 / 12.9 / 11.5 / 18.3 -> 15.5 / 11.8 / 11.5 / 18.9, 122^3 20.1 / 16.1 /
+// 15.8 / 24.7 -> 18.8 / 14.3 / 14.1 / 21.9, 180^3 49.0 / 44.0 / 41.8 / 77.4 ->
+// 47.2 / 32.9 / 30.5 / 51.0, 302^3 336 / 248 / 215 / 409 -> 273 / 175 / 136 /
+// 324; FP32 102^3 11.7 / 10.8 / 9.3 / 14.5 -> 12.1 / 10.6 / 9.4 / 15.0, 122^3
+// 14.6 / 13.2 / 11.5 / 19.0 -> 13.9 / 11.7 / 10.7 / 17.2, 302^3 203 / 165 / 144
+// / 290 -> 157 / 102 / 89 / 179.
+constexpr int kQuadMin = 112;
+
 bool dense_plan(int n, bool periodic, DensePlan* P) {
   P->n = n;
   P->periodic = periodic;
+  P->quad = periodic && n % 2 == 0 && n >= kQuadMin;
   P->R = periodic ? n : n - 1;
-  P->H = P->R / 2 + 1;
+  P->H = (P->quad ? n / 2 : P->R) / 2 + 1;
   P->MT = (P->H + 15) / 16;
   P->KS = (P->H + 7) / 8;
-  // one wave per row tile, at most 16 waves
-  return n >= 2 && P->MT <= 16;
+  // one wave per row tile, at most 16 waves (two parts)
+  return n >= 2 && P->R / 2 + 1 <= 256;
 }
 
-size_t dense_table_elems(const DensePlan& P) { return 4 * (size_t)P.MT * P.KS * 128; }
+static size_t matrix_elems(const DensePlan& P) { return (size_t)P.MT * P.KS * 128; }
+static int parts(const DensePlan& P) { return P.quad ? 4 : 2; }
 
-// The four matrices (forward even, forward odd, inverse even, inverse odd),
-// each as MT x KS fragments of 64 lanes x 2 elements: element h of lane q of
-// fragment (t, s) is M[16 t + q % 16][8 s + 4 h + q / 16], zero outside.
+size_t dense_table_elems(const DensePlan& P) { return 2 * parts(P) * matrix_elems(P); }
+
+// The matrices, forward then inverse, one per part (even, odd; QUAD: of even
+// and odd k), each as MT x KS fragments of 64 lanes x 2 elements: element h of
+// lane q of fragment (t, s) is M[16 t + q % 16][8 s + 4 h + q / 16], zero
+// outside.
 void dense_table(const DensePlan& P, double* out64, float* out32) {
-  const int n = P.n, R = P.R;
+  const int n = P.n, R = P.R, np = parts(P);
   const long mod = P.periodic ? n : 2L * R;  // angles are 2 pi m / mod
   std::vector<long double> c(mod), s(mod);
   for (long m = 0; m < mod; m++) {
@@ -478,7 +553,7 @@ void dense_table(const DensePlan& P, double* out64, float* out32) {
     if (4 * m == mod || 4 * m == 3 * mod) c[m] = 0;
     if (m == 0 || 2 * m == mod) s[m] = 0;
   }
-  const size_t msize = (size_t)P.MT * P.KS * 128;
+  const size_t msize = matrix_elems(P);
   // element (row, col) of matrix mat
   auto put = [&](int mat, int row, int col, long double v) {
     const size_t lane = (row & 15) + 16 * (col & 3);
@@ -486,19 +561,20 @@ void dense_table(const DensePlan& P, double* out64, float* out32) {
     out64[e] = (double)v;
     if (out32) out32[e] = (float)v;
   };
-  for (size_t e = 0; e < 4 * msize; e++) out64[e] = 0;
+  for (size_t e = 0; e < 2 * np * msize; e++) out64[e] = 0;
   if (out32)
-    for (size_t e = 0; e < 4 * msize; e++) out32[e] = 0;
+    for (size_t e = 0; e < 2 * np * msize; e++) out32[e] = 0;
   for (int r = 0; r < P.H; r++)  // spectral row
-    for (int odd = 0; odd < 2; odd++) {
-      const long k = P.periodic ? r : 2L * r + odd;
-      if (P.periodic ? (odd ? r < 1 || 2 * r >= n : 2 * r > n) : k >= n) continue;
-      const bool edge = P.periodic ? r == 0 || 2 * r == n : k == 0 || k == R;  // weight 1 in the inverse sum
+    for (int part = 0; part < np; part++) {
+      const bool sine = P.periodic && part >= np / 2;
+      const long k = P.quad ? 2L * r + (part & 1) : (P.periodic ? r : 2L * r + part);
+      if (P.periodic ? (sine ? k < 1 || 2 * k >= n : 2 * k > n) : k >= n) continue;
+      const bool edge = P.periodic ? k == 0 || 2 * k == n : k == 0 || k == R;  // weight 1 in the inverse sum
       long a = 0;                                                             // j * k modulo the table
       for (int j = 0; j < P.H; j++) {
-        const long double f = P.periodic && odd ? -s[a] : c[a];
-        put(odd, r, j, !P.periodic && j > 0 ? 2 * f : f);
-        put(2 + odd, j, r, edge ? f : 2 * f);
+        const long double f = sine ? -s[a] : c[a];
+        put(part, r, j, !P.periodic && j > 0 ? 2 * f : f);
+        put(np + part, j, r, edge ? f : 2 * f);
         a += k;
         if (a >= mod) a -= mod;
       }
@@ -509,7 +585,7 @@ namespace dense {
 
 size_t lds_bytes(const DensePlan& P, int axis, size_t esize) {
   const size_t kp = 8 * (size_t)P.KS;
-  return 2 * esize * NL * (axis == 0 ? kp + (esize == 8 ? Mm<double>::kPadX : Mm<float>::kPadX) : kp);
+  return parts(P) * esize * NL * (axis == 0 ? kp + (esize == 8 ? Mm<double>::kPadX : Mm<float>::kPadX) : kp);
 }
 
 }  // namespace dense
@@ -523,7 +599,7 @@ static void launch_dense_pass(const DGrid& g, const DensePlan& P, const Spectral
   const dim3 grd = AXIS == 0
                        ? dim3((unsigned)(((long)g.npts[1] * g.npts[2] + nl - 1) / nl), 1, 1)
                        : dim3((unsigned)((g.npts[0] + nl - 1) / nl), AXIS == 1 ? g.npts[2] : g.npts[1], 1);
-  auto* kernel = k_dense<T, AXIS, MODE, IO, TV>;
+  auto* kernel = P.quad ? k_dense<T, AXIS, MODE, IO, TV, true> : k_dense<T, AXIS, MODE, IO, TV, false>;
   if (lds > 64 * 1024)
     (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   // One wave per row tile; on x more, which load and store lines only.  There

@@ -46,11 +46,12 @@ struct Red3 {
 
 // One axis as products with the transform's matrices (mif_dense.hip), for
 // lengths without a specialised kernel: R is the mirror length (n, or n - 1 on
-// a Neumann axis), H = R/2 + 1 the rows of the folded line, MT and KS its
-// 16-row and 8-column tiles, M the fragment tables (null: no dense pass).
+// a Neumann axis), H = R/2 + 1 the rows of the folded line (quad, a line
+// folded twice: n/4 + 1), MT and KS its 16-row and 8-column tiles, M the
+// fragment tables (null: no dense pass).
 struct DensePlan {
   int n, R, H, MT, KS;
-  int periodic;
+  int periodic, quad;
   const double* M64;
   const float* M32;
 };
