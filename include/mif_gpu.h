@@ -320,7 +320,7 @@ int mif_field_gather_noalloc(const mif_field *f, const int32_t *ijk, int64_t n, 
  * to report the roofline of a kernel from inside a run). */
 typedef enum mif_kernel_class {
   MIF_KC_STAGE = 0,     /* fused RK3 stage (three components)              */
-  MIF_KC_BC = 1,        /* boundary shell                                   */
+  MIF_KC_BC = 1,        /* boundary shell, where not in the stage's launch  */
   MIF_KC_DIV = 2,       /* divergence -> packed right-hand side            */
   MIF_KC_FFT_X = 3,     /* x forward/inverse transform passes              */
   MIF_KC_FFT_Y = 4,     /* y forward/inverse transform passes              */
@@ -332,7 +332,8 @@ typedef enum mif_kernel_class {
   MIF_KC_FFT_X_UNPACK = 10, /* x inverse pass writing the pressure field   */
   MIF_KC_ADJOINT = 11,  /* whole adjoint step (all its kernels)            */
   MIF_KC_PRESSURE_RIM = 12, /* p += phi on the points a stage kernel with a fused
-                               projection leaves out                        */
+                               projection leaves out (no launch of its own:
+                               with the stage or the boundary shell)        */
   MIF_KC_COUNT = 13
 } mif_kernel_class;
 int mif_ctx_set_timing(mif_ctx *ctx, int enable);

@@ -150,7 +150,7 @@ constexpr int kStageSlots32 = 4, kStageSlots64 = 3;
 // rows (see the launcher)
 constexpr bool kStageVec = true;
 
-// FT (velocity-only step): MIF_FN_VT_FORCING read from the trig tables.
+// FT (velocity-only step): MIF_FN_VT_FORCING read from the axis tables.
 // VEC: halo planes fetched with 16-byte loads (element 1 of every row
 // 16-byte aligned: the layout's storage shift).
 // PROJ (kinds 2 and 3): the previous stage's projection fused in (StageArgs
