@@ -283,7 +283,11 @@ __global__ void __launch_bounds__(kAdjSumThreads) k_adj_sum(const double* __rest
 // contributions to the planes below and above.  X itself needs one plane in
 // LDS at a time, with one more halo point.  N_bar is zero outside the component
 // interiors and cells outside the arrays read as zero, so no product needs a
-// test.  76 KB of LDS, two workgroups (16 waves) per CU; the arithmetic is FP64
+// test.  Two columns read as zero too: (0, N1) and (N0, 0), where the stage
+// kernels leave what their threads outside a component's interior hold (in
+// padding of u and w, and of v), which is no finite number after a run that
+// blew up; the components that have a point there have it on an edge of the
+// domain, which no product with a nonzero factor takes.  76 KB of LDS, two workgroups (16 waves) per CU; the arithmetic is FP64
 // in both forms.  Bound by the LDS and the plane's two barriers: 128^3 FP64 153 ->
 // 99 us against gathering X and N_bar from a three-plane ring of six fields (8
 // waves per CU, 31 global taps per point); 14 words per point at 2.4 TB/s.  A
@@ -311,10 +315,12 @@ k_adj_xb(DGrid g, Layout L, AdjVec Xv, AdjVec Nbv, AdjVec Zv, AdjVec Xbv, T* __r
   const T* N[3] = {(const T*)Nbv.f[0], (const T*)Nbv.f[1], (const T*)Nbv.f[2]};
   const T* Z[3] = {(const T*)Zv.f[0], (const T*)Zv.f[1], (const T*)Zv.f[2]};
   // this thread's column, and its point of the X plane's outer ring
-  const bool own = i >= 0 && j >= 0 && i < L.PX && j < L.SY;
+  auto inside = [&](int ii, int jj) { return ii >= 0 && jj >= 0 && ii < L.PX && jj < L.SY; };
+  auto finite = [&](int ii, int jj) { return !(ii == 0 && jj == g.N[1]) && !(ii == g.N[0] && jj == 0); };
+  const bool own = inside(i, j) && finite(i, j);
   // lane offsets are 32-bit and the plane's base is uniform, so that a load
   // takes one address register
-  const unsigned oo = own ? i + L.PX * j : 0;
+  const unsigned oo = inside(i, j) ? i + L.PX * j : 0;
   int rx = 0, ry = 0;
   if (tid < AHX) {
     rx = tid;
@@ -327,7 +333,7 @@ k_adj_xb(DGrid g, Layout L, AdjVec Xv, AdjVec Nbv, AdjVec Zv, AdjVec Xbv, T* __r
   }
   const int ri = bx * AOX - 2 + rx, rj = by * AOY - 2 + ry;
   const bool ring = tid < ARING;
-  const bool rok = ring && ri >= 0 && rj >= 0 && ri < L.PX && rj < L.SY;
+  const bool rok = ring && inside(ri, rj) && finite(ri, rj);
   const unsigned ro = rok ? ri + L.PX * rj : 0;
 
   // planes outside the arrays read plane 0 and count as zero

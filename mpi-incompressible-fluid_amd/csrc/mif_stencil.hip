@@ -579,7 +579,13 @@ k_stage(DGrid g, Layout L, StageArgs s, VelStageArgs vs, ShellArg<SHELL> sh, int
             // or nothing reads (O2); threads outside the tile store at the
             // shell point (0, 0, k).  SHELL: the shell is written by this
             // launch, and both store into the padding beyond the component's
-            // extents (row N1 of u and w, column N0 of v)
+            // extents (row N1 of u and w, column N0 of v), which no reader may
+            // count on: its value is whichever thread's came last, and no
+            // number at all after a run that blew up.  (A zero there instead
+            // took the step between walls from 1036 to 1052 us per ten at 32 x
+            // 32 x 64; stores under a test of inside[c] from 990 to 1040 us at
+            // 165^3 FP64 and 806 to 854 at 193^3 mixed; an element behind the
+            // field 650 to 721 at 165^3 mixed.)
             long os = in_tile ? o : L.idx(0, 0, k);
             if constexpr (SHELL > 0) os = inside[c] ? o : (c == 1 ? L.idx(g.N[0], 0, k) : L.idx(0, g.N[1], k));
             store_out<NT>(&((T*)s.O1[c])[os], o1);
