@@ -1213,7 +1213,10 @@ int ctx_init(mif_ctx* c, const mif_grid* grid, const uint64_t Ng[3], int precisi
   }
   // the largest index the closed forms take is one past the largest extent
   c->axis_n = std::max(g.N[0], std::max(g.N[1], g.N[2])) + 2;
-  HIPCHK(nullptr, hipMalloc(&c->axis, axis_index(3, 0, 0, c->axis_n) * sizeof(double)));
+  HIPCHK(nullptr, hipMalloc(&c->axis, axis_elems(c->axis_n) * sizeof(double)));
+  const std::vector<double> es = es_axis_rows(g, c->axis_n);
+  HIPCHK(nullptr, hipMemcpy(c->axis + axis_index(0, 0, AX_EXP_A, c->axis_n), es.data(), es.size() * sizeof(double),
+                            hipMemcpyHostToDevice));
   launch_axis_tables(g, c->axis, c->axis_n, c->stream);
   LAUNCHCHK(nullptr);
   // transfers and reductions

@@ -1,6 +1,8 @@
 // mif_kernels.h -- launch interfaces of the HIP kernels (host side).
 #pragma once
 
+#include <vector>
+
 #include "mif_device.h"
 
 namespace mif {
@@ -160,7 +162,7 @@ struct BCArgs {
 struct StageShell {
   int on = 0;    // 0: a boundary pass follows the stage
   int nbx = 0;   // workgroups of a row
-  int rows = 0;  // (wall axis, component) rows; the rim's three come after them
+  int rows = 0;  // (wall axis, side, component) rows; the rim's three come after them
   BCArgs a{};
   PressureRim rim{};
   RimShape rs{};
@@ -176,8 +178,10 @@ void launch_stage(int stage, const DGrid& g, const Layout& L, const StageArgs& s
 template <typename T>
 void launch_vel_stage(int stage, const DGrid& g, const Layout& L, const VelStageArgs& s, const StageShell& sh,
                       hipStream_t st);
-// Fills the axis tables (axis_index) of n indices per axis.
+// The axis tables (axis_index) of n indices per axis: launch_axis_tables fills
+// the rows AX_SIN and AX_COS, es_axis_rows returns the others, from AX_EXP_A on.
 void launch_axis_tables(const DGrid& g, double* tab, int n, hipStream_t st);
+std::vector<double> es_axis_rows(const DGrid& g, int n);
 template <typename T>
 void launch_bc(const DGrid& g, const Layout& L, void* const F[3], const FnDesc& f, double t, hipStream_t st,
                const PressureRim& rim = PressureRim{});

@@ -744,7 +744,7 @@ __device__ inline double face_value(const DGrid& g, Ev ev, int c, int face, int 
 // from the axis tables; BC_LID the lid-driven data (one comparison); BC_FN
 // any other closed form through the general evaluator, whose serial chain of
 // FP64 transcendentals (up to ten evaluations per thread) took 30 us on 65^3
-// nodes and 25 us on 96^3 for Ethier-Steinman data (6.7 and 7.1 us from the
+// nodes and 25 us on 96^3 for Ethier-Steinman data (8 us each from the
 // tables), 63 us on 256^3 for the velocity-only field (16 us) and 12 us on
 // 32 x 32 x 64 for the lid.
 enum BCMode { BC_ZERO = 0, BC_FN = 1, BC_TABLE = 2, BC_ES = 3, BC_VT = 4, BC_LID = 5 };
@@ -810,10 +810,10 @@ __device__ inline T shell_value(const DGrid& g, const Layout& L, const BCArgs& a
   return F[L.idx(s[0], s[1], s[2])];
 }
 
-// Workgroup b of a stage's shell (StageShell), thread t of 512: two opposite
-// wall points, or a point of the pressure rim.  The points of wall axis z are
-// whole planes (ghosts of periodic axes included); those of y and x leave out
-// the wall planes that z, then y have.
+// Workgroup b of a stage's shell (StageShell), thread t of 512: a wall point,
+// or a point of the pressure rim.  The points of wall axis z are whole planes
+// (ghosts of periodic axes included); those of y and x leave out the wall
+// planes that z, then y have.
 template <typename T>
 __device__ inline void shell_block(const DGrid& g, const Layout& L, const StageShell& sh, int b, int t) {
   const int row = b / sh.nbx;
@@ -823,8 +823,8 @@ __device__ inline void shell_block(const DGrid& g, const Layout& L, const StageS
                    sh.rs.imax, sh.rs.jmax, sh.rs.kmax);
     return;
   }
-  const int c = row % 3;
-  int wall = row / 3, axis = 2;
+  const int c = row % 3, side = row / 3 & 1;
+  int wall = row / 6, axis = 2;
   for (int a = 2; a >= 0; a--)
     if (!g.periodic[a] && wall-- == 0) axis = a;
   int e[3];
@@ -836,21 +836,18 @@ __device__ inline void shell_block(const DGrid& g, const Layout& L, const StageS
   if (q >= (long)n0 * n1) return;
   const int q0 = lo0 + (int)(q % n0), q1 = lo1 + (int)(q / n0);
   T* F = (T*)sh.a.F[c];
-#pragma unroll 1
-  for (int side = 0; side < 2; side++) {
-    const int w = side ? e[axis] - 1 : 0;
-    const int i = axis == 0 ? w : q0, j = axis == 1 ? w : (axis == 0 ? q0 : q1), k = axis == 2 ? w : q1;
-    T v;
-    if (sh.a.f.kind == MIF_FN_ZERO)
-      v = (T)0;
-    else if (sh.a.f.kind == MIF_FN_ES_VELOCITY)
-      v = shell_value<T, BC_ES>(g, L, sh.a, c, e, i, j, k, F);
-    else if (sh.a.f.kind == MIF_FN_VT_VELOCITY)
-      v = shell_value<T, BC_VT>(g, L, sh.a, c, e, i, j, k, F);
-    else
-      v = shell_value<T, BC_LID>(g, L, sh.a, c, e, i, j, k, F);
-    F[L.idx(i, j, k)] = v;
-  }
+  const int w = side ? e[axis] - 1 : 0;
+  const int i = axis == 0 ? w : q0, j = axis == 1 ? w : (axis == 0 ? q0 : q1), k = axis == 2 ? w : q1;
+  T v;
+  if (sh.a.f.kind == MIF_FN_ZERO)
+    v = (T)0;
+  else if (sh.a.f.kind == MIF_FN_ES_VELOCITY)
+    v = shell_value<T, BC_ES>(g, L, sh.a, c, e, i, j, k, F);
+  else if (sh.a.f.kind == MIF_FN_VT_VELOCITY)
+    v = shell_value<T, BC_VT>(g, L, sh.a, c, e, i, j, k, F);
+  else
+    v = shell_value<T, BC_LID>(g, L, sh.a, c, e, i, j, k, F);
+  F[L.idx(i, j, k)] = v;
 }
 
 // Each thread owns the two opposite shell points of one (pair, position):
@@ -976,10 +973,13 @@ template <typename T, typename S, int NHN>
 __global__ void __launch_bounds__(256) k_div_rhs(DGrid g, Layout L, const T* __restrict__ u, const T* __restrict__ v,
                                                  const T* __restrict__ w, S* __restrict__ B, long bp0, long bplane,
                                                  double dt, FnDesc gp, double tg) {
-  const int a = blockIdx.x * blockDim.x + threadIdx.x;  // packed owner coordinates
-  const int b = blockIdx.y;
+  // packed owner coordinates; NHN 3: a wave takes 8 x 8 points, so that eight
+  // rows share the evaluation that a single lane of each row on an x wall asks for
+  const int t = threadIdx.x;
+  const int a = NHN == 3 ? 32 * blockIdx.x + 8 * (t >> 6) + (t & 7) : 256 * blockIdx.x + t;
+  const int b = NHN == 3 ? 8 * blockIdx.y + (t >> 3 & 7) : blockIdx.y;
   const int c = blockIdx.z;
-  if (a >= g.npts[0]) return;
+  if (a >= g.npts[0] || (NHN == 3 && b >= g.npts[1])) return;
   const int i = a + g.olo[0], j = b + g.olo[1], k = c + g.olo[2];
   const long o = L.idx(i, j, k);
   const double du_dx = ((double)u[o + 1] - (double)u[o]) * g.one_over_h[0];
@@ -988,14 +988,18 @@ __global__ void __launch_bounds__(256) k_div_rhs(DGrid g, Layout L, const T* __r
   double r = (du_dx + dv_dy + dw_dz) / dt;
   if (NHN == 3) {
     // the Ethier-Steinman gradient from the axis tables, tg its time factor
-    // (65^3 nodes: 48 -> 6 us against the general evaluator)
+    // (65^3 nodes: 48 us by the general evaluator, 9.7 here; 96^3: 17.2 us with
+    // 64 points of a row to a wave, 14.9 with 16 x 4, 13.6 with 8 x 8; 193^3:
+    // 84 and 69 us with the last two)
     const AxisEval at{gp.axis, gp.an, 3, {i, j, k}};
-    if (k == 0) r += at.es_grad_p(2, 0, 1) * tg * 2.0 * g.one_over_h[2];
-    if (k == g.N[2] - 1) r -= at.es_grad_p(2, 0, 1) * tg * 2.0 * g.one_over_h[2];
-    if (j == 0) r += at.es_grad_p(1, 2, 0) * tg * 2.0 * g.one_over_h[1];
-    if (j == g.N[1] - 1) r -= at.es_grad_p(1, 2, 0) * tg * 2.0 * g.one_over_h[1];
-    if (i == 0) r += at.es_grad_p(0, 1, 2) * tg * 2.0 * g.one_over_h[0];
-    if (i == g.N[0] - 1) r -= at.es_grad_p(0, 1, 2) * tg * 2.0 * g.one_over_h[0];
+    const int sk = k == 0 ? 1 : (k == g.N[2] - 1 ? -1 : 0), sj = j == 0 ? 1 : (j == g.N[1] - 1 ? -1 : 0),
+              si = i == 0 ? 1 : (i == g.N[0] - 1 ? -1 : 0);
+    if (sk || sj || si) {
+      const AxisEval::GradParts t = at.es_grad_parts();
+      if (sk) r += sk * at.es_grad_p(t, 2, 0, 1) * tg * 2.0 * g.one_over_h[2];
+      if (sj) r += sj * at.es_grad_p(t, 1, 2, 0) * tg * 2.0 * g.one_over_h[1];
+      if (si) r += si * at.es_grad_p(t, 0, 1, 2) * tg * 2.0 * g.one_over_h[0];
+    }
   } else if (NHN == 1) {
     const int sx = g.N[0], sy = g.N[1], sz = g.N[2];
     if (k == 0) r += eval_at(g, gp, 3, 2, tg, i, j, k) * 2.0 * g.one_over_h[2];
@@ -1393,7 +1397,7 @@ StageShell stage_shell(const DGrid& g, const Layout& L, bool full_step, void* co
   long mx = 0;
   for (int a = 0; a < 3; a++) {
     if (g.periodic[a]) continue;
-    sh.rows += 3;
+    sh.rows += 6;
     const int a0 = a == 0 ? 1 : 0, a1 = a == 2 ? 1 : 2;
     mx = max(mx, (long)(g.N[a0] + 1) * (g.N[a1] + 1));
   }
@@ -1457,13 +1461,30 @@ __global__ void __launch_bounds__(256) k_axis_tables(DGrid g, double* __restrict
   const int a = blockIdx.y / 2, sh = blockIdx.y % 2;
   if (i >= n) return;
   const double x = coord(g, a, sh ? a : 3, i);
-  const double xa = MIF_PI / 4 * x, xd = MIF_PI / 2 * x;
-  const double v[kAxisFns] = {sin(x), cos(x), exp(xa), sin(xa), cos(xa), sin(xd), cos(xd)};
-  for (int f = 0; f < kAxisFns; f++) tab[axis_index(a, sh, f, n) + i] = v[f];
+  tab[axis_index(a, sh, AX_SIN, n) + i] = sin(x);
+  tab[axis_index(a, sh, AX_COS, n) + i] = cos(x);
 }
 
 void launch_axis_tables(const DGrid& g, double* tab, int n, hipStream_t st) {
   k_axis_tables<<<dim3((n + 255) / 256, 6, 1), 256, 0, st>>>(g, tab, n);
+}
+
+std::vector<double> es_axis_rows(const DGrid& g, int n) {
+  const long first = axis_index(0, 0, AX_EXP_A, n);
+  std::vector<double> rows(axis_elems(n) - first);
+  for (int a = 0; a < 3; a++)
+    for (int sh = 0; sh < 2; sh++)
+      for (int i = 0; i < n; i++) {
+        const long double x = (long double)(MIF_PI / 4) * coord(g, a, sh ? a : 3, i);
+        const long double s = sinl(x), c = cosl(x);
+        const long double v[kAxisLow] = {expl(x), s, c, 2 * s * c, (c - s) * (c + s)};
+        for (int f = 0; f < kAxisLow; f++) {
+          const double h = (double)v[f];
+          rows[axis_index(a, sh, AX_EXP_A + f, n) - first + i] = h;
+          rows[axis_index(a, sh, kAxisFns + f, n) - first + i] = (double)(v[f] - h);
+        }
+      }
+  return rows;
 }
 
 static void shell_counts(const DGrid& g, int stag, int cnt[3]) {
@@ -1539,13 +1560,14 @@ template <typename T, typename S>
 void launch_div_rhs(const DGrid& g, const Layout& L, const T* u, const T* v, const T* w, S* B, long bp0, long bplane,
                     double dt, const FnDesc& gp, double tg, int nhn, hipStream_t st) {
   dim3 grd((g.npts[0] + 255) / 256, g.npts[1], g.npts[2]);
+  const dim3 grd3((g.npts[0] + 31) / 32, (g.npts[1] + 7) / 8, g.npts[2]);
   if (nhn && gp.kind == kFnFaceTable)
     k_div_rhs<T, S, 2><<<grd, 256, 0, st>>>(g, L, u, v, w, B, bp0, bplane, dt, gp, tg);
   else if (nhn && gp.kind == MIF_FN_ES_GRAD_P)
-    k_div_rhs<T, S, 3><<<grd, 256, 0, st>>>(g, L, u, v, w, B, bp0, bplane, dt, gp, time_factor(gp.kind, tg, gp.Re));
+    k_div_rhs<T, S, 3><<<grd3, 256, 0, st>>>(g, L, u, v, w, B, bp0, bplane, dt, gp, time_factor(gp.kind, tg, gp.Re));
   else if (nhn && gp.kind == MIF_FN_TIME_DIFFERENCE && gp.base == MIF_FN_ES_GRAD_P)
-    k_div_rhs<T, S, 3><<<grd, 256, 0, st>>>(g, L, u, v, w, B, bp0, bplane, dt, gp,
-                                            grad_p_factor_difference(gp.t1, gp.t0, gp.Re));
+    k_div_rhs<T, S, 3><<<grd3, 256, 0, st>>>(g, L, u, v, w, B, bp0, bplane, dt, gp,
+                                             grad_p_factor_difference(gp.t1, gp.t0, gp.Re));
   else if (nhn)
     k_div_rhs<T, S, 1><<<grd, 256, 0, st>>>(g, L, u, v, w, B, bp0, bplane, dt, gp, tg);
   else
