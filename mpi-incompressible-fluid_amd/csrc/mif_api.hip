@@ -672,11 +672,12 @@ int stage(mif_ctx* c, int st, mif_field* const X[3], mif_field* const A[3], mif_
   PressureRim rim;
   if (phi) rim = PressureRim{p, phi, pout, c->phi_mean};
   const StageShell sh = stage_shell(c->g, c->L, true, s.O1, f, t, rim);
+  bool shell;
   {
     KTimer tm(c, MIF_KC_STAGE);
-    launch_stage<T>(st, c->g, c->L, s, sh, c->stream);
+    shell = launch_stage<T>(st, c->g, c->L, s, sh, c->stream);
   }
-  if (!sh.on) apply_bc<T>(c, O1, f, t, rim);
+  if (!shell) apply_bc<T>(c, O1, f, t, rim);
   if (phi) c->phi_mean = nullptr;
   return MIF_OK;
 }
@@ -841,11 +842,12 @@ int velocity_timestep(mif_ctx* c, mif_field* const vel[3], mif_field* const buf[
     }
     s.t = t;
     const StageShell sh = stage_shell(c->g, c->L, false, F, ev[n - 1], t_bc, PressureRim{});
+    bool shell;
     {
       KTimer tm(c, MIF_KC_STAGE);
-      launch_vel_stage<T>(n, c->g, c->L, s, sh, c->stream);
+      shell = launch_vel_stage<T>(n, c->g, c->L, s, sh, c->stream);
     }
-    if (!sh.on) apply_bc<T>(c, out, ev[n - 1], t_bc);
+    if (!shell) apply_bc<T>(c, out, ev[n - 1], t_bc);
   };
   run(1, vel, t_n, buf, time_1);
   run(2, buf, time_1, vel, time_2);

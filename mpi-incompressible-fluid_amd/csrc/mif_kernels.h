@@ -160,7 +160,7 @@ struct BCArgs {
 // periodic images too, and `rows` + 3 rows of nbx further workgroups fill the
 // wall faces and the rim.
 struct StageShell {
-  int on = 0;    // 0: a boundary pass follows the stage
+  int on = 0;    // 0: not wanted
   int nbx = 0;   // workgroups of a row
   int rows = 0;  // (wall axis, side, component) rows; the rim's three come after them
   BCArgs a{};
@@ -172,11 +172,13 @@ struct StageShell {
 StageShell stage_shell(const DGrid& g, const Layout& L, bool full_step, void* const F[3], const FnDesc& f, double t,
                        const PressureRim& rim);
 
+// A stage, and the shell sh with it where there is a kernel for the two: false
+// if not, and a boundary pass has to follow.
 template <typename T>
-void launch_stage(int stage, const DGrid& g, const Layout& L, const StageArgs& s, const StageShell& sh,
+bool launch_stage(int stage, const DGrid& g, const Layout& L, const StageArgs& s, const StageShell& sh,
                   hipStream_t st);
 template <typename T>
-void launch_vel_stage(int stage, const DGrid& g, const Layout& L, const VelStageArgs& s, const StageShell& sh,
+bool launch_vel_stage(int stage, const DGrid& g, const Layout& L, const VelStageArgs& s, const StageShell& sh,
                       hipStream_t st);
 // The axis tables (axis_index) of n indices per axis: launch_axis_tables fills
 // the rows AX_SIN and AX_COS, es_axis_rows returns the others, from AX_EXP_A on.

@@ -1304,7 +1304,7 @@ static int stage_chunk(long cols, int planes, int most) {
 }
 
 template <typename T, int KIND, bool FT = false, bool NT = false>
-static void launch_stage_kind(const DGrid& g, const Layout& L, const StageArgs& s, const VelStageArgs& vs,
+static bool launch_stage_kind(const DGrid& g, const Layout& L, const StageArgs& s, const VelStageArgs& vs,
                               const StageShell& sh, hipStream_t st) {
   // union of the three components' interiors
   int eu[3], ev[3], ew[3];
@@ -1328,11 +1328,21 @@ static void launch_stage_kind(const DGrid& g, const Layout& L, const StageArgs& 
     k_stage<T, KIND, FT, NT, V, P, S><<<ntiles + nshell, blk, 0, st>>>(g, L, s, vs, arg, imax, jmax, kmax, ntx, nty,
                                                                       ntiles, kchunk);
   };
+  // whether the shell is written too: periodic axes have kernels for it on
+  // small grids (stage_shell) only, the full step's with ordinary accesses
   auto go = [&](auto vec, auto proj) {
-    if (!sh.on) return run(vec, proj, std::integral_constant<int, 0>{});
-    if (!g.periodic[0] && !g.periodic[1] && !g.periodic[2]) return run(vec, proj, std::integral_constant<int, 1>{});
-    // stage_shell: full step, small grids
-    if constexpr (!NT && KIND <= 3) run(vec, proj, std::integral_constant<int, 2>{});
+    const bool images = g.periodic[0] || g.periodic[1] || g.periodic[2];
+    if (sh.on && !images) {
+      run(vec, proj, std::integral_constant<int, 1>{});
+      return true;
+    }
+    if constexpr (!NT && KIND <= 3)
+      if (sh.on) {
+        run(vec, proj, std::integral_constant<int, 2>{});
+        return true;
+      }
+    run(vec, proj, std::integral_constant<int, 0>{});
+    return false;
   };
   using yes = std::true_type;
   using no = std::false_type;
@@ -1362,7 +1372,7 @@ static void launch_stage_kind(const DGrid& g, const Layout& L, const StageArgs& 
   if constexpr (kFuse) {
     if (s.phi) return go(no{}, yes{});
   }
-  go(no{}, no{});
+  return go(no{}, no{});
 }
 
 // The launch saved against what the stage kernel loses by it.  Without a
@@ -1413,15 +1423,17 @@ StageShell stage_shell(const DGrid& g, const Layout& L, bool full_step, void* co
 }
 
 template <typename T>
-void launch_stage(int stage, const DGrid& g, const Layout& L, const StageArgs& s, const StageShell& sh,
+bool launch_stage(int stage, const DGrid& g, const Layout& L, const StageArgs& s, const StageShell& sh,
                   hipStream_t st) {
   VelStageArgs vs{};
   if (stage == 1)
-    L.nt ? launch_stage_kind<T, 1, false, true>(g, L, s, vs, sh, st) : launch_stage_kind<T, 1>(g, L, s, vs, sh, st);
-  else if (stage == 2)
-    L.nt ? launch_stage_kind<T, 2, false, true>(g, L, s, vs, sh, st) : launch_stage_kind<T, 2>(g, L, s, vs, sh, st);
-  else
-    L.nt ? launch_stage_kind<T, 3, false, true>(g, L, s, vs, sh, st) : launch_stage_kind<T, 3>(g, L, s, vs, sh, st);
+    return L.nt ? launch_stage_kind<T, 1, false, true>(g, L, s, vs, sh, st)
+                : launch_stage_kind<T, 1>(g, L, s, vs, sh, st);
+  if (stage == 2)
+    return L.nt ? launch_stage_kind<T, 2, false, true>(g, L, s, vs, sh, st)
+                : launch_stage_kind<T, 2>(g, L, s, vs, sh, st);
+  return L.nt ? launch_stage_kind<T, 3, false, true>(g, L, s, vs, sh, st)
+              : launch_stage_kind<T, 3>(g, L, s, vs, sh, st);
 }
 
 // The velocity-only kinds read 6 to 9 arrays and write 3 to 6, and are bound by
@@ -1435,25 +1447,21 @@ void launch_stage(int stage, const DGrid& g, const Layout& L, const StageArgs& s
 constexpr long kVelNtMinFieldBytes = 40L << 20;
 
 template <typename T>
-void launch_vel_stage(int stage, const DGrid& g, const Layout& L, const VelStageArgs& vs, const StageShell& sh,
+bool launch_vel_stage(int stage, const DGrid& g, const Layout& L, const VelStageArgs& vs, const StageShell& sh,
                       hipStream_t st) {
   StageArgs s{};
   auto go = [&](auto ft, auto nt) {
     constexpr bool F = decltype(ft)::value, N = decltype(nt)::value;
-    if (stage == 1)
-      launch_stage_kind<T, 4, F, N>(g, L, s, vs, sh, st);
-    else if (stage == 2)
-      launch_stage_kind<T, 5, F, N>(g, L, s, vs, sh, st);
-    else
-      launch_stage_kind<T, 6, F, N>(g, L, s, vs, sh, st);
+    if (stage == 1) return launch_stage_kind<T, 4, F, N>(g, L, s, vs, sh, st);
+    if (stage == 2) return launch_stage_kind<T, 5, F, N>(g, L, s, vs, sh, st);
+    return launch_stage_kind<T, 6, F, N>(g, L, s, vs, sh, st);
   };
   using yes = std::true_type;
   using no = std::false_type;
   const bool nt = L.nt && L.elems * (long)sizeof(T) > kVelNtMinFieldBytes;
   if (vs.forcing.kind == MIF_FN_VT_FORCING)
-    nt ? go(yes{}, yes{}) : go(yes{}, no{});
-  else
-    nt ? go(no{}, yes{}) : go(no{}, no{});
+    return nt ? go(yes{}, yes{}) : go(yes{}, no{});
+  return nt ? go(no{}, yes{}) : go(no{}, no{});
 }
 
 __global__ void __launch_bounds__(256) k_axis_tables(DGrid g, double* __restrict__ tab, int n) {
@@ -1672,8 +1680,8 @@ void launch_gather(const Layout& L, const T* F, const int* ijk, long n, double* 
 }
 
 #define MIF_INSTANTIATE(T)                                                                                          \
-  template void launch_stage<T>(int, const DGrid&, const Layout&, const StageArgs&, const StageShell&, hipStream_t); \
-  template void launch_vel_stage<T>(int, const DGrid&, const Layout&, const VelStageArgs&, const StageShell&,       \
+  template bool launch_stage<T>(int, const DGrid&, const Layout&, const StageArgs&, const StageShell&, hipStream_t); \
+  template bool launch_vel_stage<T>(int, const DGrid&, const Layout&, const VelStageArgs&, const StageShell&,       \
                                     hipStream_t);                                                                   \
   template void launch_bc<T>(const DGrid&, const Layout&, void* const*, const FnDesc&, double, hipStream_t,         \
                              const PressureRim&);                                                                   \
