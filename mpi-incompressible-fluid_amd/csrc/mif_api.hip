@@ -14,6 +14,7 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <type_traits>
 #include <unordered_set>
 #include <vector>
 
@@ -375,15 +376,19 @@ int spectral_solve(mif_ctx* c, T* B) {
 template <typename T, typename TF>
 int solve_into_field(mif_ctx* c, T* B, mif_field* p, bool pack) {
   const SpectralScale sc = scale_of<T>(c);
+  static_assert(sizeof(TF) <= sizeof(T), "the x inverse pass writes a field of its own precision or FP32");
+  // the x forward pass reads a field of its own precision only
+  const bool from_field = pack && std::is_same_v<T, TF> && fused_x_pass(c->plan[0]);
+  if (pack && !from_field) launch_pack<TF, T>(c->g, c->L, fptr<TF>(p), B, c->bp0, c->bplane, c->stream);
   if (fused_x_pass(c->plan[0])) {
     FusedIO io{};
     io.P = p->data;
     io.L = c->L;
     io.fields_fp32 = sizeof(T) == 8 && sizeof(TF) == 4;
-    io.pack = pack;
+    io.pack = from_field;
     {
       KTimer t(c, MIF_KC_FFT_X);
-      if (pack)
+      if (from_field)
         launch_fused_x<T>(c->g, 0, c->plan[0], sc, B, c->bp0, c->bplane, io, c->stream);
       else
         launch_fft_axis<T>(c->g, 0, -1, 0, c->plan[0], sc, B, c->bp0, c->bplane, c->stream);
@@ -392,7 +397,6 @@ int solve_into_field(mif_ctx* c, T* B, mif_field* p, bool pack) {
     KTimer t(c, MIF_KC_FFT_X_UNPACK);
     launch_fused_x<T>(c->g, 1, c->plan[0], sc, B, c->bp0, c->bplane, io, c->stream);
   } else {
-    if (pack) launch_pack<TF, T>(c->g, c->L, fptr<TF>(p), B, c->bp0, c->bplane, c->stream);
     const int rc = spectral_solve<T>(c, B);
     if (rc) return rc;
     KTimer t(c, MIF_KC_UNPACK);
