@@ -335,15 +335,15 @@ void spectral_middle(mif_ctx* c, T* B) {
   const SpectralScale sc = scale_of<T>(c);
   {
     KTimer t(c, MIF_KC_FFT_Y);
-    launch_fft_axis<T>(c->g, 1, -1, 0, c->plan[1], sc, B, c->bp0, c->bplane, c->stream);
+    launch_fft_axis<T>(c->g, 1, -1, c->plan[1], sc, B, c->bp0, c->bplane, c->stream);
   }
   {
     KTimer t(c, MIF_KC_FFT_Z);
-    launch_fft_axis<T>(c->g, 2, 0, 1, c->plan[2], sc, B, c->bp0, c->bplane, c->stream);
+    launch_fft_axis<T>(c->g, 2, 0, c->plan[2], sc, B, c->bp0, c->bplane, c->stream);
   }
   {
     KTimer t(c, MIF_KC_FFT_Y);
-    launch_fft_axis<T>(c->g, 1, +1, 0, c->plan[1], sc, B, c->bp0, c->bplane, c->stream);
+    launch_fft_axis<T>(c->g, 1, +1, c->plan[1], sc, B, c->bp0, c->bplane, c->stream);
   }
 }
 
@@ -357,12 +357,12 @@ int spectral_solve(mif_ctx* c, T* B) {
   const SpectralScale sc = scale_of<T>(c);
   {
     KTimer t(c, MIF_KC_FFT_X);
-    launch_fft_axis<T>(c->g, 0, -1, 0, c->plan[0], sc, B, c->bp0, c->bplane, c->stream);
+    launch_fft_axis<T>(c->g, 0, -1, c->plan[0], sc, B, c->bp0, c->bplane, c->stream);
   }
   spectral_middle<T>(c, B);
   {
     KTimer t(c, MIF_KC_FFT_X);
-    launch_fft_axis<T>(c->g, 0, +1, 0, c->plan[0], sc, B, c->bp0, c->bplane, c->stream);
+    launch_fft_axis<T>(c->g, 0, +1, c->plan[0], sc, B, c->bp0, c->bplane, c->stream);
   }
   LAUNCHCHK(c);
   return MIF_OK;
@@ -391,7 +391,7 @@ int solve_into_field(mif_ctx* c, T* B, mif_field* p, bool pack) {
       if (from_field)
         launch_fused_x<T>(c->g, 0, c->plan[0], sc, B, c->bp0, c->bplane, io, c->stream);
       else
-        launch_fft_axis<T>(c->g, 0, -1, 0, c->plan[0], sc, B, c->bp0, c->bplane, c->stream);
+        launch_fft_axis<T>(c->g, 0, -1, c->plan[0], sc, B, c->bp0, c->bplane, c->stream);
     }
     spectral_middle<T>(c, B);
     KTimer t(c, MIF_KC_FFT_X_UNPACK);
@@ -583,7 +583,7 @@ int pressure_solve_mixed_dc1(mif_ctx* c, mif_field* p, mif_field* const vel[3], 
   spectral_middle<float>(c, B32);
   {
     KTimer t(c, MIF_KC_FFT_X);
-    launch_fft_axis<float>(c->g, 0, +1, 0, c->plan[0], sc, B32, c->bp0, c->bplane, c->stream);
+    launch_fft_axis<float>(c->g, 0, +1, c->plan[0], sc, B32, c->bp0, c->bplane, c->stream);
   }
   {
     // the x forward pass forms the defect as it loads its lines

@@ -383,9 +383,9 @@ static void launch_one(const DGrid& g, const FftPlan& plan, const SpectralScale&
 }
 
 template <typename T>
-void launch_fft_axis(const DGrid& g, int axis, int dir, int fused, const FftPlan& plan, const SpectralScale& sc, T* B,
+void launch_fft_axis(const DGrid& g, int axis, int dir, const FftPlan& plan, const SpectralScale& sc, T* B,
                      long bp0, long bplane, hipStream_t st) {
-  const int mode = fused ? 2 : (dir < 0 ? 0 : 1);
+  const int mode = axis == 2 ? 2 : (dir < 0 ? 0 : 1);
   if (plan.dct2) {
     // cell-centred axes: y only, lengths with a kernel (checked when the
     // context is created)
@@ -446,9 +446,9 @@ template void launch_fused_x<double>(const DGrid&, int, const FftPlan&, const Sp
                                      const FusedIO&, hipStream_t);
 template void launch_fused_x<float>(const DGrid&, int, const FftPlan&, const SpectralScale&, float*, long, long,
                                     const FusedIO&, hipStream_t);
-template void launch_fft_axis<double>(const DGrid&, int, int, int, const FftPlan&, const SpectralScale&, double*, long,
+template void launch_fft_axis<double>(const DGrid&, int, int, const FftPlan&, const SpectralScale&, double*, long,
                                       long, hipStream_t);
-template void launch_fft_axis<float>(const DGrid&, int, int, int, const FftPlan&, const SpectralScale&, float*, long,
+template void launch_fft_axis<float>(const DGrid&, int, int, const FftPlan&, const SpectralScale&, float*, long,
                                      long, hipStream_t);
 
 }  // namespace mif

@@ -1097,9 +1097,7 @@ static void launch_p2(const DGrid& g, int axis, int mode, const FftPlan& plan, c
       if (mode == 0) MIF_P2(1, 0);
       else MIF_P2(1, 1);
     } else if (axis == 2) {
-      if (mode == 0) MIF_P2(2, 0);
-      else if (mode == 1) MIF_P2(2, 1);
-      else MIF_P2(2, 2);
+      MIF_P2(2, 2);
     }
   }
 #undef MIF_P2

@@ -233,21 +233,22 @@ void launch_norm_pressure(const DGrid& g, const Layout& L, const T* p, const FnD
                           const ExactTables& tab, Red3* partial, int nblocks, Red3* out, hipStream_t st);
 
 // Spectral solve passes on the packed buffer B (extents npts, row pitch bp0,
-// plane pitch bplane).  dir: -1 forward, +1 inverse; axis 2 with fused = 1
-// runs forward, scale, inverse in one pass.
+// plane pitch bplane).  dir: -1 forward, +1 inverse on axes 0 and 1; axis 2 has
+// one pass only, forward, scaling and inverse, whatever dir is.
 template <typename T>
-void launch_fft_axis(const DGrid& g, int axis, int dir, int fused, const FftPlan& plan, const SpectralScale& sc, T* B,
+void launch_fft_axis(const DGrid& g, int axis, int dir, const FftPlan& plan, const SpectralScale& sc, T* B,
                      long bp0, long bplane, hipStream_t st);
 // Specialised transform pass (complex lengths 2^k and 3 * 2^k, see
 // fft_fast_len); on axis 0 with io set, the forward pass is fused with the
 // divergence (mode 0) and the inverse with the unpack into the pressure field
-// (mode 1).  Returns false when the length has no specialised kernel.
+// (mode 1); axis 2 is mode 2, forward, scaling and inverse.  Returns false when
+// the length has no specialised kernel.
 bool fft_fast_len(int L);
 template <typename T>
 bool launch_fft_pow2(const DGrid& g, int axis, int mode, const FftPlan& plan, const SpectralScale& sc, T* B, long bp0,
                      long bplane, const FusedIO* io, hipStream_t st);
 // The passes as matrix products (mif_dense.hip): axis 0 with mode 0 / 1 (io
-// as in launch_fft_pow2), axis 1 with mode 0 / 1, axis 2 with mode 2.
+// as in launch_fft_pow2), axis 1 with mode 0 / 1, axis 2 is mode 2.
 // dense_plan fills the tile counts (false: the line is too long).
 bool dense_plan(int n, bool periodic, DensePlan* P);
 // The fragment tables of a plan: dense_table_elems elements, in FP64 and (out32
