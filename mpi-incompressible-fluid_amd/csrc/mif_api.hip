@@ -1038,9 +1038,7 @@ int upload_face_tables(mif_ctx* c, bool velocity, const double* host, int count,
 // x axis short enough for dense_x_short.
 bool dense_axis(int axis, const FftPlan& P) {
   if (P.dct2 || P.L < 2) return false;
-  if (fft_fast_len(P.L)) return axis == 0 && P.L <= 128;
-  // the half-length DCT-I of long wall-normal y axes
-  return !(axis == 1 && !P.periodic && (P.L == 1024 || P.L == 1536 || P.L == 2048));
+  return !fft_fast_len(P.L) || (axis == 0 && P.L <= 128);
 }
 
 // Constants, layout, transform plans and scratch of a new context.

@@ -26,9 +26,13 @@
 // between walls, FP64 406 / 407 / 806 -> 17 / 16 / 26; 201^3, FP64 150 / 164 /
 // 294 -> 65 / 59 / 111, FP32 115 / 132 / 234 -> 42 / 41 / 77; 256^3, FP64 629 /
 // 645 / 1220 -> 116 / 109 / 208; 480 x 480 x 199 points, periodic, FP64 661 /
-// 675 / 13572 -> 531 / 516 / 538.  It was faster at every length measured
-// from 20 to 481, smooth or not, so every length that one workgroup's 16
-// waves can hold takes it (dense_plan); longer ones stay with mif_fft.hip.
+// 675 / 13572 -> 531 / 516 / 538.  It was faster at every length measured,
+// smooth or not, 2 to 24 points with 256 on the other axes (whole solve, walls
+// / periodic, FP64: 2 points 167 -> 42 / 39 -> 28 us, 16 points 226 -> 56 / 81
+// -> 43; up to 8 times in FP32) and 20 to 481 on all, so every line whose row
+// tiles in two parts one workgroup's 16 waves can hold takes it: up to 512 wall
+// nodes or 511 periodic points (dense_plan).  Longer ones stay with mif_fft.hip,
+// also the even periodic ones that four parts would hold.
 // At 256 nodes the products take 4.3 GFLOP per pass (about 55 us at the FP64
 // rate) and the memory 60 us: the two phases of a workgroup overlap only
 // through the other three workgroups of its CU.
@@ -526,7 +530,8 @@ bool dense_plan(int n, bool periodic, DensePlan* P) {
   P->H = (P->quad ? n / 2 : P->R) / 2 + 1;
   P->MT = (P->H + 15) / 16;
   P->KS = (P->H + 7) / 8;
-  // one wave per row tile, at most 16 waves (two parts)
+  // one wave per row tile, at most 16 waves in two parts (longer lines in four
+  // parts have not been measured)
   return n >= 2 && P->R / 2 + 1 <= 256;
 }
 
