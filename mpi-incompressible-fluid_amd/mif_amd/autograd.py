@@ -8,8 +8,10 @@ steps, and records the three stencil sources of every step of the last
 interval (u^n and the two stage buffers) as it runs them.  backward runs the
 hand-written adjoint of each step (mif_timestep_adjoint) in reverse: the last
 interval from the forward's records, every earlier one after replaying it
-once from its checkpoint.  Memory: one (u, p) per checkpoint plus 3 velocity
-triples per step of one interval.
+once from its checkpoint.  The forward runs those intervals with fused
+projections and the replay without; the states are the same bit for bit.
+Memory: one (u, p) per checkpoint plus 3 velocity triples per step of one
+interval.
 
 No counterpart in the reference (it has no adjoint); the forward map is the
 reference's timestep() (src/Timestep.cpp:97-156) with a body force added to
@@ -100,20 +102,25 @@ class Rollout:
         try:
             if is_callables(self.ev):
                 for s in range(s0, s0 + n):
-                    timestep(self.vel, self.buf, self.buf2, self.ev, s * self.ctx.dt, self.p, self.pb)
+                    timestep(self.vel, self.buf, self.buf2, self.ev, self._time(s, s0), self.p, self.pb)
             else:
                 timestep_n(self.vel, self.buf, self.buf2, self.ev, s0 * self.ctx.dt, self.p, self.pb, n)
         finally:
             self.ctx.set_stage_records(True)
 
     # -- forward / backward -----------------------------------------------------
+    def _time(self, s: int, s0: int):
+        """Time of step s of the interval from step s0, rounded as timestep_n
+        does, so that the replay's states are the forward's bit for bit."""
+        return s0 * self.ctx.dt + (s - s0) * self.ctx.dt
+
     def _record_step(self, s: int, s0: int):
         # timestep() leaves Y2 and Y3 (after their projections) in its two
         # buffers, so the recorded triples serve as the buffers; only u^n,
         # which the step overwrites, is copied
         un, y2, y3 = self.rec[s - s0]
         un.copy_from(self.vel)
-        timestep(self.vel, y2, y3, self.ev, s * self.ctx.dt, self.p, self.pb)
+        timestep(self.vel, y2, y3, self.ev, self._time(s, s0), self.p, self.pb)
 
     def run_forward(self, u0, f):
         self.generation += 1
