@@ -19,6 +19,7 @@ the momentum right-hand side.
 """
 from __future__ import annotations
 
+import contextlib
 import time
 
 import torch
@@ -98,15 +99,12 @@ class Rollout:
         """n steps from step s0 that need no records: in one call, their
         projections fused into the stage kernels (75 words per unknown and
         step instead of 96)."""
-        self.ctx.set_stage_records(False)
-        try:
+        with self._records(False):
             if is_callables(self.ev):
                 for s in range(s0, s0 + n):
                     timestep(self.vel, self.buf, self.buf2, self.ev, self._time(s, s0), self.p, self.pb)
             else:
                 timestep_n(self.vel, self.buf, self.buf2, self.ev, s0 * self.ctx.dt, self.p, self.pb, n)
-        finally:
-            self.ctx.set_stage_records(True)
 
     # -- forward / backward -----------------------------------------------------
     def _time(self, s: int, s0: int):
@@ -114,13 +112,25 @@ class Rollout:
         does, so that the replay's states are the forward's bit for bit."""
         return s0 * self.ctx.dt + (s - s0) * self.ctx.dt
 
+    @contextlib.contextmanager
+    def _records(self, keep: bool):
+        """The context's stage records as the rollout's steps need them; its
+        other users find their own setting again."""
+        before = self.ctx.stage_records
+        self.ctx.set_stage_records(keep)
+        try:
+            yield
+        finally:
+            self.ctx.set_stage_records(before)
+
     def _record_step(self, s: int, s0: int):
         # timestep() leaves Y2 and Y3 (after their projections) in its two
         # buffers, so the recorded triples serve as the buffers; only u^n,
         # which the step overwrites, is copied
         un, y2, y3 = self.rec[s - s0]
         un.copy_from(self.vel)
-        timestep(self.vel, y2, y3, self.ev, self._time(s, s0), self.p, self.pb)
+        with self._records(True):
+            timestep(self.vel, y2, y3, self.ev, self._time(s, s0), self.p, self.pb)
 
     def run_forward(self, u0, f):
         self.generation += 1

@@ -105,6 +105,7 @@ class Context:
         _check(self.lib.mif_ctx_info(self.ptr, ctypes.byref(dt), ext), self.ptr)
         self.dt = dt.value
         self.node_extents = tuple(int(e) for e in ext)
+        self.stage_records = False
         self._fields = weakref.WeakSet()
 
     def close(self):
@@ -158,6 +159,7 @@ class Context:
         two buffers (what timestep_adjoint reads); otherwise the projections
         of stages 1 and 2 are fused into the next stage kernel (the default)."""
         self.check(self.lib.mif_ctx_set_stage_records(self.ptr, 1 if keep else 0))
+        self.stage_records = bool(keep)
 
     def set_body_force(self, f):
         """Constant body force added to N in every stage of timestep()

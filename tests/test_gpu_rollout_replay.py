@@ -42,3 +42,34 @@ def test_replay_ends_at_the_next_checkpoint(Ng, per, kind, form):
                         [*roll.cp_u[c + 1].download(), roll.cp_p[c + 1].download()]):
             assert np.array_equal(a, b)
     ctx.close()
+
+
+def test_the_context_keeps_its_own_records_setting():
+    """A context that other steps use with fused projections keeps them so, and
+    the rollout's gradient does not depend on the setting."""
+    print("[case] rollout leaves the stage records setting", flush=True)
+    grads, fields = [], []
+    for keep in (True, False):
+        ctx, roll, u0 = rollout((17, 20, 19), (0, 0, 0), "fp64", mif.FN_ZERO)
+        ctx.set_stage_records(keep)
+        us = [t.clone().requires_grad_(True) for t in u0]
+        f = torch.zeros(3, dtype=torch.float64, requires_grad=True)
+        out = roll(us, f)
+        grads.append(torch.autograd.grad(sum((t * t).sum() for t in out), [*us, f]))
+        vel, buf, buf2, p, pb = ctx.velocity(), ctx.velocity(), ctx.velocity(), ctx.pressure(), ctx.pressure()
+        vel.upload([t.cpu().numpy() for t in u0])
+        mif.timestep(vel, buf, buf2, roll.ev, 0.0, p, pb)
+        fields.append(buf.download())
+        if not keep:  # what a context without a rollout leaves in its buffer
+            fresh = mif.Context(ctx.grid)
+            v, b, b2, q, qb = (fresh.velocity(), fresh.velocity(), fresh.velocity(), fresh.pressure(),
+                               fresh.pressure())
+            v.upload([t.cpu().numpy() for t in u0])
+            mif.timestep(v, b, b2, roll.ev, 0.0, q, qb)
+            for x, y in zip(buf.download(), b.download()):
+                assert np.array_equal(x, y)
+            fresh.close()
+        ctx.close()
+    for a, b in zip(*grads):
+        assert torch.equal(a, b)
+    assert not np.array_equal(fields[0][0], fields[1][0])
