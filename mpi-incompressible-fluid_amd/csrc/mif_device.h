@@ -152,24 +152,28 @@ __host__ __device__ inline double vt_forcing(int c, double sx, double cx, double
 }
 
 // Kept out of line: the closed forms are large and only the boundary,
-// forcing and set-up kernels evaluate them.
-__device__ __noinline__ double fn_base(const FnDesc& f, int kind, int c, double t, double x, double y, double z) {
+// forcing and set-up kernels evaluate them.  Of a descriptor it takes Re: a
+// reference would have every thread copy the kernel's argument to scratch
+// first (240 to 336 bytes: a 128^3 FP64 field set to zero 118 -> 17 us, to the
+// Ethier-Steinman u 120 -> 30, 257^3 boundary pass of the PT field 52 -> 41,
+// velocity-only step at 128^3 with constant forcing 403 -> 196).
+__device__ __noinline__ double fn_base(int kind, int c, double t, double x, double y, double z, double Re) {
   switch (kind) {
     case MIF_FN_ZERO:
       return 0.0;
     case MIF_FN_ES_VELOCITY:
-      return c == 0 ? es_u(t, x, y, z, f.Re) : (c == 1 ? es_u(t, y, z, x, f.Re) : es_u(t, z, x, y, f.Re));
+      return c == 0 ? es_u(t, x, y, z, Re) : (c == 1 ? es_u(t, y, z, x, Re) : es_u(t, z, x, y, Re));
     case MIF_FN_ES_PRESSURE:
-      return es_p(t, x, y, z, f.Re);
+      return es_p(t, x, y, z, Re);
     case MIF_FN_ES_GRAD_P:
-      return c == 0 ? es_dpdx(t, x, y, z, f.Re) : (c == 1 ? es_dpdx(t, y, z, x, f.Re) : es_dpdx(t, z, x, y, f.Re));
+      return c == 0 ? es_dpdx(t, x, y, z, Re) : (c == 1 ? es_dpdx(t, y, z, x, Re) : es_dpdx(t, z, x, y, Re));
     case MIF_FN_VT_VELOCITY:
       // generators/manufsol_velocity.py:55-57
       if (c == 0) return sin(x) * cos(y) * sin(z) * sin(t);
       if (c == 1) return cos(x) * sin(y) * sin(z) * sin(t);
       return 2 * cos(x) * cos(y) * cos(z) * sin(t);
     case MIF_FN_VT_FORCING:
-      return vt_forcing(c, sin(x), cos(x), sin(y), cos(y), sin(z), cos(z), sin(t), cos(t), f.Re);
+      return vt_forcing(c, sin(x), cos(x), sin(y), cos(y), sin(z), cos(z), sin(t), cos(t), Re);
     case MIF_FN_PT_VELOCITY:
     case MIF_FN_PT_GRAD_P:
       // generators/manufsol_pressure.py:36-38 (grad p equals the velocity)
@@ -186,17 +190,20 @@ __device__ __noinline__ double fn_base(const FnDesc& f, int kind, int c, double 
       const double eps = 1e-12;
       return (c == 1 && x < xl + eps && x > xl - eps) ? 1.0 : 0.0;
     }
-    case MIF_FN_CONSTANT:
-      return f.c[c];
     default:
       return 0.0;
   }
 }
 
 __device__ inline double fn_eval(const FnDesc& f, int c, double t, double x, double y, double z) {
-  if (f.kind == MIF_FN_TIME_DIFFERENCE)
-    return fn_base(f, f.base, c, f.t1, x, y, z) - fn_base(f, f.base, c, f.t0, x, y, z);
-  return fn_base(f, f.kind, c, t, x, y, z);
+  const bool difference = f.kind == MIF_FN_TIME_DIFFERENCE;
+  const int kind = difference ? f.base : f.kind;
+  if (kind == MIF_FN_CONSTANT) {
+    const double k = c == 0 ? f.c[0] : (c == 1 ? f.c[1] : f.c[2]);
+    return difference ? k - k : k;
+  }
+  const double v = fn_base(kind, c, difference ? f.t1 : t, x, y, z, f.Re);
+  return difference ? v - fn_base(kind, c, f.t0, x, y, z, f.Re) : v;
 }
 
 // Coordinate of index i along axis a for staggering s: min + h*(base+i),
