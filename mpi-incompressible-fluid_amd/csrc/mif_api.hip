@@ -87,7 +87,7 @@ struct mif_ctx {
   double kappa = 0;
   // spectral solve
   FftPlan plan[3]{};
-  unsigned char* tables = nullptr;  // every axis table of the solve, one allocation
+  unsigned char* tables = nullptr;  // every table of an axis, one allocation
   const double* lam[3]{};
   double inv_norm = 1;
   long bp0 = 0, bplane = 0, belems = 0;
@@ -118,7 +118,7 @@ struct mif_ctx {
   double* adj_fbar = nullptr;
   bool adj_ready = false;  // every adjoint buffer allocated
   // functions of one coordinate that the boundary data, the forcing and the
-  // Neumann data are built from (launch_axis_tables)
+  // Neumann data are built from (axis_index), in `tables`
   double* axis = nullptr;
   int axis_n = 0;
   // transfers and reductions
@@ -1206,6 +1206,9 @@ int ctx_init(mif_ctx* c, const mif_grid* grid, const uint64_t Ng[3], int precisi
     // the DCT-III of a cell-centred axis returns n times the line
     norm *= (double)(Ng[a] - 1) * (g.periodic[a] || g.cell[a] ? 1.0 : 2.0);
   }
+  // the largest index the closed forms take is one past the largest extent
+  c->axis_n = std::max(g.N[0], std::max(g.N[1], g.N[2])) + 2;
+  add_table(&c->axis, es_axis_tables(g, c->axis_n));
   HIPCHK(nullptr, hipMalloc(&c->tables, tab.size()));
   HIPCHK(nullptr, hipMemcpy(c->tables, tab.data(), tab.size(), hipMemcpyHostToDevice));
   for (const auto& e : at) *e.first = c->tables + e.second;
@@ -1215,12 +1218,6 @@ int ctx_init(mif_ctx* c, const mif_grid* grid, const uint64_t Ng[3], int precisi
     c->nxpart = fused_x_blocks(g, c->plan[0], false);
     if (c->nxpart > 0) HIPCHK(nullptr, hipMalloc(&c->xpart, c->nxpart * sizeof(Red3)));
   }
-  // the largest index the closed forms take is one past the largest extent
-  c->axis_n = std::max(g.N[0], std::max(g.N[1], g.N[2])) + 2;
-  HIPCHK(nullptr, hipMalloc(&c->axis, axis_elems(c->axis_n) * sizeof(double)));
-  const std::vector<double> es = es_axis_rows(g, c->axis_n);
-  HIPCHK(nullptr, hipMemcpy(c->axis + axis_index(0, 0, AX_EXP_A, c->axis_n), es.data(), es.size() * sizeof(double),
-                            hipMemcpyHostToDevice));
   launch_axis_tables(g, c->axis, c->axis_n, c->stream);
   LAUNCHCHK(nullptr);
   // transfers and reductions
@@ -1351,7 +1348,6 @@ int mif_ctx_destroy(mif_ctx* c) {
   (void)hipFree(c->ftab);
   (void)hipFree(c->adj_partial);
   (void)hipFree(c->adj_fbar);
-  (void)hipFree(c->axis);
   (void)hipFree(c->tables);
   (void)hipFree(c->staging);
   (void)hipFree(c->partial);

@@ -180,10 +180,11 @@ bool launch_stage(int stage, const DGrid& g, const Layout& L, const StageArgs& s
 template <typename T>
 bool launch_vel_stage(int stage, const DGrid& g, const Layout& L, const VelStageArgs& s, const StageShell& sh,
                       hipStream_t st);
-// The axis tables (axis_index) of n indices per axis: launch_axis_tables fills
-// the rows AX_SIN and AX_COS, es_axis_rows returns the others, from AX_EXP_A on.
+// The axis tables (axis_index) of n indices per axis: es_axis_tables returns
+// them with the rows AX_SIN and AX_COS empty, which launch_axis_tables fills on
+// the device.
+std::vector<double> es_axis_tables(const DGrid& g, int n);
 void launch_axis_tables(const DGrid& g, double* tab, int n, hipStream_t st);
-std::vector<double> es_axis_rows(const DGrid& g, int n);
 template <typename T>
 void launch_bc(const DGrid& g, const Layout& L, void* const F[3], const FnDesc& f, double t, hipStream_t st,
                const PressureRim& rim = PressureRim{});
