@@ -157,12 +157,13 @@ struct BCArgs {
 };
 // The boundary pass and the pressure rim of a stage, in the stage's own
 // launch: the stage kernel stores its boundary-adjacent points at their
-// periodic images too, and `rows` + 3 rows of nbx further workgroups fill the
-// wall faces and the rim.
+// periodic images too, and further workgroups fill the wall faces and the rim.
 struct StageShell {
   int on = 0;    // 0: not wanted
-  int nbx = 0;   // workgroups of a row
-  int rows = 0;  // (wall axis, side, component) rows; the rim's three come after them
+  // workgroups of a row: of each axis (0: no wall), whose rows are (side,
+  // component), and of the rim, whose rows are its three groups
+  int nb[3] = {}, nb_rim = 0;
+  int blocks() const { return 6 * (nb[0] + nb[1] + nb[2]) + 3 * nb_rim; }
   BCArgs a{};
   PressureRim rim{};
   RimShape rs{};

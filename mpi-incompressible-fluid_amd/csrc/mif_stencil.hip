@@ -816,17 +816,22 @@ __device__ inline T shell_value(const DGrid& g, const Layout& L, const BCArgs& a
 // planes that z, then y have.
 template <typename T>
 __device__ inline void shell_block(const DGrid& g, const Layout& L, const StageShell& sh, int b, int t) {
-  const int row = b / sh.nbx;
-  const long q = (long)(b - row * sh.nbx) * 512 + t;
-  if (row >= sh.rows) {
-    p_rim_point<T>(g, L, row - sh.rows, q, (const T*)sh.rim.pin, (const T*)sh.rim.phi, (T*)sh.rim.pout, sh.rim.mean,
+  // (every count read first, so that they are chosen as values: as conditional
+  // reads the compiler turned them into one read through a chosen address and
+  // lost the rim's)
+  const int nx = sh.nb[0], ny = sh.nb[1], nz = sh.nb[2], nr = sh.nb_rim;
+  const int y0 = 6 * nx, z0 = y0 + 6 * ny, r0 = z0 + 6 * nz;
+  const int axis = (b >= y0) + (b >= z0) + (b >= r0);  // 3: the rim
+  const int nb = axis == 0 ? nx : (axis == 1 ? ny : (axis == 2 ? nz : nr));
+  b -= axis == 0 ? 0 : (axis == 1 ? y0 : (axis == 2 ? z0 : r0));
+  const int row = b / nb;
+  const long q = (long)(b - row * nb) * 512 + t;
+  if (axis == 3) {
+    p_rim_point<T>(g, L, row, q, (const T*)sh.rim.pin, (const T*)sh.rim.phi, (T*)sh.rim.pout, sh.rim.mean,
                    sh.rs.imax, sh.rs.jmax, sh.rs.kmax);
     return;
   }
-  const int c = row % 3, side = row / 3 & 1;
-  int wall = row / 6, axis = 2;
-  for (int a = 2; a >= 0; a--)
-    if (!g.periodic[a] && wall-- == 0) axis = a;
+  const int c = row % 3, side = row / 3;
   int e[3];
   extents(g, c, e);
   // the two other axes: ranges [lo, lo + n)
@@ -1322,7 +1327,7 @@ static bool launch_stage_kind(const DGrid& g, const Layout& L, const StageArgs& 
     constexpr int S = decltype(shell)::value;
     const int kchunk = stage_chunk(ntx * nty, kmax, stage_planes<T, KIND, NT, P>());
     const int ntiles = ntx * nty * ((kmax + kchunk - 1) / kchunk);
-    const int nshell = S > 0 ? sh.nbx * (sh.rows + (sh.rim.pin ? 3 : 0)) : 0;
+    const int nshell = S > 0 ? sh.blocks() : 0;
     ShellArg<S> arg;
     if constexpr (S > 0) arg = sh;
     k_stage<T, KIND, FT, NT, V, P, S><<<ntiles + nshell, blk, 0, st>>>(g, L, s, vs, arg, imax, jmax, kmax, ntx, nty,
@@ -1404,12 +1409,10 @@ StageShell stage_shell(const DGrid& g, const Layout& L, bool full_step, void* co
   if (images ? !full_step || (long)g.N[0] * g.N[1] * g.N[2] > kShellMaxPoints : full_step && L.elems > kShellMaxElems)
     return sh;
   sh.on = 1;
-  long mx = 0;
   for (int a = 0; a < 3; a++) {
     if (g.periodic[a]) continue;
-    sh.rows += 6;
     const int a0 = a == 0 ? 1 : 0, a1 = a == 2 ? 1 : 2;
-    mx = max(mx, (long)(g.N[a0] + 1) * (g.N[a1] + 1));
+    sh.nb[a] = (int)(((long)(g.N[a0] + 1) * (g.N[a1] + 1) + 511) / 512);
   }
   for (int c = 0; c < 3; c++) sh.a.F[c] = F[c];
   sh.a.f = f;
@@ -1417,8 +1420,7 @@ StageShell stage_shell(const DGrid& g, const Layout& L, bool full_step, void* co
   if (f.kind == MIF_FN_ES_VELOCITY || f.kind == MIF_FN_VT_VELOCITY) sh.a.tf = time_factor(f.kind, t, f.Re);
   sh.rim = rim;
   sh.rs = rim_shape(g);
-  if (rim.pin) mx = max(mx, max(sh.rs.count[0], max(sh.rs.count[1], sh.rs.count[2])));
-  sh.nbx = (int)((mx + 511) / 512);
+  if (rim.pin) sh.nb_rim = (int)((max(sh.rs.count[0], max(sh.rs.count[1], sh.rs.count[2])) + 511) / 512);
   return sh;
 }
 
